@@ -157,8 +157,8 @@ int rk_mm_int4_g128(const void* X, int x_dtype, int ldx, const uint8_t* q, const
  * fragment order, then blocks of 128 / 64 / 48 rows x 128 columns fed by direct memory-to-LDS copies; chosen when
  * the shape has enough column blocks to fill the chip, K is short enough for a block's scale and min rows to sit
  * in LDS, and N * K / 128 is a multiple of 8; RK_MM_WIDE128 is the same for M > 64 with K / 128 even and >= 4:
- * 128 x 128 blocks of four waves, each owning 64 x 64 of the block, two blocks per CU, split over K (*splits > 1)
- * for M >= 256 with K / 128 > 16 when the tiles are few), or, for
+ * blocks of 128 columns and 96 or 128 rows, a wave per 32 columns, two blocks per CU or one block whose waves share
+ * the groups two ways; split over K (*splits > 1) for M > 128 with K / 128 > 16 when the tiles are few), or, for
  * M <= 48 and K <= 2048 (with or without a workspace),
  * RK_MM_STREAM (X held in registers as matrix-core fragments for the whole launch while 16-column tiles of codes
  * stream past, one block per CU, no workspace);

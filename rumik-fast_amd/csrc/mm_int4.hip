@@ -12,6 +12,7 @@
 //   * per group: C = sum of 4 MFMAs from zero, then acc = scale * C + xsum * min in fp32 (xsum[g][m] precomputed
 //     per block in LDS; a lane's 4 D rows are 4 consecutive m, one ds_read_b128).
 // Codes never leave int4 in HBM; every product is exact, sums are fp32.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -414,7 +415,9 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
 // Xp[mt][g][t][lane] (16 bytes): afrag of X[16 mt + j][128 g + 32 s + 8 t .. + 7], lane = j + 16 s (rows past M are
 // zero); xs[g][m] = fp32 sum of X[m][128 g .. 128 g + 127]. One thread per 16-byte chunk (m, g, c = 4 s + t); block
 // b = (m tile, group) covers the 16 rows' 16 chunks of one group, so it writes one whole 4 KiB fragment block.
-template <bool BF16>
+// X32: the fragment order of the 32 x 32 x 16 MFMAs of mm_int4_wide_kernel instead: chunk c = 8 h + t of row m sits at
+// Xp[m / 16][g][t][h][m % 16].
+template <bool BF16, bool X32>
 __global__ __launch_bounds__(256) void mm_xprep_kernel(const void* __restrict__ X, int ldx, int M, int Mp, int K,
                                                        uint4* __restrict__ Xp, float* __restrict__ xs) {
     const int NG = K >> 7;
@@ -423,8 +426,8 @@ __global__ __launch_bounds__(256) void mm_xprep_kernel(const void* __restrict__ 
     u4_t d = {0u, 0u, 0u, 0u};
     if (m < M)
         d = *reinterpret_cast<const u4_t*>(reinterpret_cast<const uint16_t*>(X) + (size_t)m * ldx + 128 * g + 8 * c);
-    const int s = c >> 2, t = c & 3;
-    Xp[(((size_t)(m >> 4) * NG + g) * 4 + t) * 64 + (m & 15) + 16 * s] =
+    const int slot = X32 ? 2 * (c & 7) + (c >> 3) : 4 * (c & 3) + (c >> 2);  // of the block's 16 rows
+    Xp[((size_t)(m >> 4) * NG + g) * 256 + 16 * slot + (m & 15)] =
         __builtin_bit_cast(uint4, afrag(d, BF16 ? RK_BF16 : RK_F16));
     float f = 0.f;
     if (BF16) {
@@ -617,27 +620,35 @@ RK_PREP_INST(8)
 #undef RK_PREP_INST
 
 // ------------------------------------------------------------------------------- prepared-X kernel, wide waves
-// mm_int4_wide_kernel: the prepared X of mm_xprep_kernel, blocks of 128 rows x 128 columns with four waves in a
-// 2 x 2 layout, wave (wm, wn) owning rows 64 wm .. + 63 and columns 64 wn .. + 63 (4 x 4 MFMA tiles), two blocks
-// per CU:
-//   * each X fragment read from LDS feeds four MFMAs (the fragment reads set the pace of the one-column-tile
-//     layout); each code column is dequantised by the two waves that share it;
-//   * codes go straight into registers, two steps ahead; X copies go into a two-slot LDS ring with
+// mm_int4_wide_kernel: the prepared X of mm_xprep_kernel<., true>, blocks of 32 MT rows x 128 columns. A wave owns 32
+// columns for all of the block's rows (MT MFMA tiles of 32 x 32); four waves per K way, KW K ways (K way kw takes
+// every KW-th group; the ways' sums meet in LDS at the end). KW = 1: two blocks per CU, which pass their barriers
+// independently, so one block's affine, waits and barrier overlap the other's MFMAs. KW = 2, one block per CU, when
+// the shape has no more blocks than CUs: the same eight waves per CU on half the steps.
+//   * what bounds it is instruction issue: a 16 x 16 x 32 MFMA holds its 16 cycles but also takes ~9 cycles of the
+//     SIMD's VALU issue, a 32 x 32 x 16 MFMA ~13 of its 32 (measured with one MFMA and one VALU wave per SIMD), so
+//     the larger tile leaves 60% of the time to VALU work instead of 40%; and a wave that owns its columns alone
+//     dequantises each code once (the 64 x 64 layout did it twice): 72 conversion ops per 32 MFMAs, and one scale
+//     per lane and step;
+//   * codes go straight into registers, two steps ahead; X copies go into a two-step LDS ring with
 //     global_load_lds, one barrier per step;
 //   * the min term sum_g xs[m][g] min[n][g] is each accumulator's starting value, computed on the matrix cores in
-//     fp32 (v_mfma_f32_16x16x4f32, four groups per instruction) while the first copies land, from row sums copied
-//     into the ring slot that step 0 leaves free; the per-step affine is one FMA per output (scale);
-//   * the two blocks of a CU pass their barriers independently, so one block's affine, waits and barrier overlap
-//     the other block's MFMAs.
-// The ring slot of step g + 1 is filled after the barrier of step g, which every wave passes only once it has
-// left step g - 1 (the slot's previous step).
-constexpr int kWideRing = 2;
-constexpr int kWideSlot = 8 * 4 * 64 * 16;              // one step's X fragments: 8 m tiles x 4 MFMA steps
-constexpr int kWideOut = 4 * 64 * 65 * 4;               // epilogue transpose, per wave [64][65] fp32
-constexpr int kWideArea = kWideOut > kWideRing * kWideSlot ? kWideOut : kWideRing * kWideSlot;
+//     fp32 (v_mfma_f32_32x32x2f32, two groups per instruction) while the first copies land, from row sums copied
+//     into the ring slot that step 0 leaves free; the per-step affine is one FMA per output (scale).
+// The ring slot of step s + 1 is filled after the barrier of step s, which every wave passes only once it has
+// left step s - 1 (the slot's previous step).
+// Operand layout of v_mfma_f32_32x32x16_f16: A[i][k] lane i + 32 (k / 8) element k % 8, B[k][j] lane j + 32 (k / 8),
+// D[i][j] lane j + 32 ((i / 4) % 2) element 4 (i / 8) + i % 4. Lane half h = lane / 32 holds columns 64 h .. + 63 of
+// the group (8 per MFMA t), so a lane's codes are 32 consecutive bytes of its column.
+constexpr int kWideCols = 128;
+constexpr int wide_slot_bytes(int MT) { return MT * 8 * 64 * 16; }  // one group's X fragments: MT tiles x 8 MFMA steps
+constexpr int wide_area_bytes(int MT, int KW) {  // the ring, reused for the waves' [32 MT][33] fp32 output tiles
+    return std::max(2 * KW * wide_slot_bytes(MT), 4 * KW * 32 * MT * 33 * 4);
+}
 
 // ngs: the most groups one block takes (its split of K)
-size_t mm_wide_lds_bytes(int ngs) { return (size_t)kWideArea + (size_t)2 * 128 * ngs * 2; }
+template <int MT, int KW>
+size_t mm_wide_lds_bytes(int ngs) { return (size_t)wide_area_bytes(MT, KW) + (size_t)2 * kWideCols * ngs * 2; }
 
 // split sp of `splits` over the K / 128 groups, in whole pairs of groups: first group and count
 __host__ __device__ inline void wide_split(int NG, int splits, int sp, int& g_lo, int& ngs) {
@@ -661,38 +672,41 @@ RK_DEV void wide_barrier() {
 // its fp32 partial sums to part[split][M][N] (mm_splitk_reduce adds them in split order); with splits = 1 it takes
 // all groups and writes Y. Requires K / 128 even, every split's group count >= 4 and <= kWideMaxGroups, and 4-byte
 // aligned scale / min arrays; the host checks all of them.
-constexpr int kWideMaxGroups = 26;  // LDS: 2 x 128 x 26 fp16 of tables beside the 66.5 KiB area stays <= 80 KiB
+constexpr int kWideMaxGroups = 26;  // LDS: 2 x 128 x 26 fp16 of tables beside the 66 KiB area (KW = 1) stay <= 80 KiB
 
-__global__ __launch_bounds__(256, 2) void mm_int4_wide_kernel(const uint4* __restrict__ Xp,
+template <int MT, int KW>
+__global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))) void mm_int4_wide_kernel(const uint4* __restrict__ Xp,
                                                               const float* __restrict__ xsg, int Mp,
                                                               const uint8_t* __restrict__ q,
                                                               const uint16_t* __restrict__ sc,
                                                               const uint16_t* __restrict__ mn, void* __restrict__ Y,
                                                               int ydt, int ldy, int M, int N, int K, int splits) {
-    constexpr int BM = 128;
+    constexpr int BM = 32 * MT, BN = kWideCols, CW = 4, SLOT = wide_slot_bytes(MT);
+    constexpr int XC = MT * 8 / CW;  // X copies of a wave per step (its K way's slot is copied by the way's four waves)
     extern __shared__ __align__(16) uint8_t smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave & 1, wn = wave >> 1;
+    const int cw = wave % CW, kw = wave / CW;
     // 1-D grid, XCD-grouped: the row blocks of one column block (and split) run on one L2
     const int G = gridDim.x, L = blockIdx.x, GY = (Mp + BM - 1) / BM;
     const int Lv = (G % 8 == 0) ? (L % 8) * (G / 8) + L / 8 : L;
     const int T = G / splits, sp = Lv / T, tl = Lv - sp * T;
-    const int mb = (tl % GY) * BM, nb = (tl / GY) * 128;
+    const int mb = (tl % GY) * BM, nb = (tl / GY) * BN;
     const int NG = K >> 7;
     int g_lo, ngs;  // this block's groups g_lo .. g_lo + ngs - 1
     wide_split(NG, splits, sp, g_lo, ngs);
-    const int mts = min(8, (Mp - mb) >> 4);  // m tiles of this block present in Xp
-    uint16_t* tsc = reinterpret_cast<uint16_t*>(smem + kWideArea);  // [128][ngs]
-    uint16_t* tmn = tsc + 128 * ngs;
-    float* xsl = reinterpret_cast<float*>(smem + kWideSlot);  // row sums [g][128] in ring slot 1 until step 0
-    const int jn = lane & 15, sq = lane >> 4;
+    const int ns = ngs / KW;  // steps: K way kw computes the block's groups KW s + kw
+    const int mts = min(2 * MT, (Mp - mb) >> 4);  // 16-row tiles of this block present in Xp
+    uint16_t* tsc = reinterpret_cast<uint16_t*>(smem + wide_area_bytes(MT, KW));  // [BN][ngs]
+    uint16_t* tmn = tsc + BN * ngs;
+    float* xsl = reinterpret_cast<float*>(smem + KW * SLOT);  // row sums [g][BM] in the ring's second step until step 0
+    const int jn = lane & 31, hf = lane >> 5;
 
     // the block's scale and min entries ([n][g] for its groups: 4-byte copies, as g_lo and NG are even; columns
     // past N repeat the last) and row sums
     {
-        const int hw = ngs >> 1, nd = 128 * hw;  // dwords per column, per table
-        for (int b0 = wave * 64; b0 < nd; b0 += 256) {
+        const int hw = ngs >> 1, nd = BN * hw;  // dwords per column, per table
+        for (int b0 = wave * 64; b0 < nd; b0 += 256 * KW) {
             const int i = b0 + lane, c = i / hw, d = i - c * hw;
             const size_t src = ((size_t)min(nb + c, N - 1) * NG + g_lo) / 2 + d;
             if (i < nd) {
@@ -702,45 +716,45 @@ __global__ __launch_bounds__(256, 2) void mm_int4_wide_kernel(const uint4* __res
                                                  reinterpret_cast<uint32_t*>(tmn) + b0, 4, 0, 0);
             }
         }
-        // xs[g][mb .. mb + 127] (rows past Mp repeat its last 4: their sums are never stored), 32 chunks a group
-        for (int b0 = wave * 64; b0 < 32 * ngs; b0 += 256) {
-            const int c = b0 + lane, g = c >> 5, r4 = min(c & 31, 4 * mts - 1);
-            if (c < 32 * ngs)
+        // xs[g][mb .. mb + BM - 1] (rows past Mp repeat its last 4: their sums are never stored), BM / 4 chunks a group
+        for (int b0 = wave * 64; b0 < BM / 4 * ngs; b0 += 256 * KW) {
+            const int c = b0 + lane, g = c / (BM / 4), r4 = min(c - g * (BM / 4), 4 * mts - 1);
+            if (c < BM / 4 * ngs)
                 __builtin_amdgcn_global_load_lds(
                     reinterpret_cast<const uint4*>(xsg + (size_t)(g_lo + g) * Mp + mb) + r4,
                     reinterpret_cast<uint4*>(xsl) + b0, 16, 0, 0);
         }
     }
-    // step g's X fragments i = wave + 4 k (m tile i / 4, MFMA step t = i % 4) into ring slot `sl`
-    auto issue_x = [&](int g, int sl) {
-        uint4* slot = reinterpret_cast<uint4*>(smem + (size_t)sl * kWideSlot);
+    // step s's X fragments i = cw + CW k of this wave's K way (32-row tile i / 8, MFMA step t = i % 8) into the ring;
+    // a lane's row lies in 16-row tile 2 (i / 8) + (lane / 16) % 2 (tiles past Mp repeat the last: their rows are
+    // never stored)
+    auto issue_x = [&](int st, int rs) {  // step, ring position
+        uint4* slot = reinterpret_cast<uint4*>(smem + (size_t)(rs * KW + kw) * SLOT);
+        const size_t g = g_lo + (size_t)st * KW + kw;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int i = wave + 4 * k, mt = i >> 2, t = i & 3;
+        for (int k = 0; k < XC; ++k) {
+            const int i = cw + CW * k, mt = i >> 3, t = i & 7;
+            const int m16 = min(2 * mt + ((lane >> 4) & 1), mts - 1);
             __builtin_amdgcn_global_load_lds(
-                Xp + (((size_t)(mb / 16 + min(mt, mts - 1)) * NG + g_lo + g) * 4 + t) * 64 + lane,
-                slot + (mt * 4 + t) * 64, 16, 0, 0);
+                Xp + ((size_t)(mb / 16 + m16) * NG + g) * 256 + 32 * t + 16 * hf + (lane & 15),
+                slot + (mt * 8 + t) * 64, 16, 0, 0);
         }
     };
-    // this lane's code bytes: column nb + 64 wn + 16 nt + jn (clamped), bytes 16 sq .. + 15 of each group. The
+    // this lane's code bytes: column nb + 32 cw + jn (clamped), bytes 32 hf .. + 31 of each group. The
     // addresses pass through a volatile asm statement, which stays behind the X copies issued before it, so the
     // code loads follow those copies (the wait counts rely on that order; plain loads of read-only memory would
     // otherwise be free to move ahead of them).
-    const uint8_t* wsrc[4];
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) wsrc[nt] = q + (size_t)min(nb + 64 * wn + 16 * nt + jn, N - 1) * (size_t)(K >> 1) + 16 * sq;
+    const uint8_t* wsrc = q + (size_t)min(nb + 32 * cw + jn, N - 1) * (size_t)(K >> 1) + 32 * hf;
     using gu4 = const __attribute__((address_space(1))) u4_t;
-    auto load_w = [&](int g, u4_t (&w)[4]) {
-        uint64_t a[4];
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) a[nt] = (uint64_t)(wsrc[nt] + 64 * (g_lo + g));
-        asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
-#pragma unroll
-        for (int nt = 0; nt < 4; ++nt) w[nt] = *(gu4*)a[nt];
+    auto load_w = [&](int st, u4_t (&w)[2]) {
+        uint64_t a = (uint64_t)(wsrc + 64 * ((size_t)g_lo + (size_t)st * KW + kw));
+        asm volatile("" : "+v"(a));
+        w[0] = *(gu4*)a;
+        w[1] = *(gu4*)(a + 16);
     };
 
     issue_x(0, 0);
-    u4_t wa[4], wb[4];  // codes of the even / odd steps
+    u4_t wa[2], wb[2];  // codes of the even / odd steps
     load_w(0, wa);
     load_w(1, wb);
     // the epilogue's arguments come in before the loop (a scalar load in flight would turn the loop's LDS waits
@@ -748,113 +762,112 @@ __global__ __launch_bounds__(256, 2) void mm_int4_wide_kernel(const uint4* __res
     asm volatile("" ::: "memory");
     asm volatile("" ::"s"(Y), "s"(ydt), "s"(ldy), "s"(M), "s"(N));
 
-    // the min term as the accumulators' start: tables and row sums landed (older than the 16 loads above)
-    wide_barrier<16>();
-    f4_t acc[4][4];
+    // the min term as the accumulators' start: tables and row sums landed (older than the loads above)
+    wide_barrier<XC + 4>();
+    f16_t acc[MT];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) acc[mt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
-    for (int qq = 0; qq < ngs; qq += 4) {
-        const int gl = qq + sq;
-        float mv[4], xa[4];
+        for (int e = 0; e < 16; ++e) acc[mt][e] = 0.f;
+    const uint16_t* scol = tsc + (32 * cw + jn) * ngs + kw;
+    const uint16_t* mcol = tmn + (32 * cw + jn) * ngs + kw;
+    for (int p = 0; p < ns; p += 2) {
+        const int st = p + hf;
+        const float mv = st < ns ? f16_bits_to_f32(mcol[st * KW]) : 0.f;
+        float xa[MT];
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) mv[nt] = gl < ngs ? f16_bits_to_f32(tmn[(64 * wn + 16 * nt + jn) * ngs + gl]) : 0.f;
+        for (int mt = 0; mt < MT; ++mt) xa[mt] = st < ns ? xsl[(st * KW + kw) * BM + 32 * mt + jn] : 0.f;
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) xa[mt] = gl < ngs ? xsl[gl * 128 + 64 * wm + 16 * mt + jn] : 0.f;
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[mt], mv[nt], acc[mt][nt], 0, 0, 0);
+        for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[mt], mv, acc[mt], 0, 0, 0);
     }
 
     const DqConsts kc = {opaque(0x000F000Fu), opaque(0x00F000F0u), opaque(0x64006400u)};
-    // one K step (slot sl = g % 2): this wave's codes of step g are in w; on return they hold step g + 2's. Every
-    // step issues the same loads in the same order (the last steps repeat the last group's, into the free slot and
-    // the consumed registers), so one wait count fits every step: when step g starts, the loads newer than its X
-    // copies and codes are step g + 1's codes (4 loads).
-    auto step = [&](int g, int sl, u4_t (&w)[4], auto last) {
-        wide_barrier<4>();
-        if constexpr (!decltype(last)::value) issue_x(min(g + 1, ngs - 1), sl ^ 1);  // into step g - 1's slot
-        const uint4* slot = reinterpret_cast<const uint4*>(smem + (size_t)sl * kWideSlot);
-        h8_t A[4][4];  // the wave's 4 m tiles x 4 MFMA steps
+    // one K step: this wave's codes of step st are in w; on return they hold step st + 2's. Every step issues the same
+    // loads in the same order (the last steps repeat the last group's, into the free slot and the consumed
+    // registers), so one wait count fits every step: when step st starts, the loads newer than its X copies and
+    // codes are step st + 1's codes (2 loads).
+    auto step = [&](int st, u4_t (&w)[2], auto last) {
+        constexpr bool kLast = decltype(last)::value;
+        wide_barrier<2>();
+        if constexpr (!kLast) issue_x(min(st + 1, ns - 1), (st + 1) & 1);  // into step st - 1's slot
+        const uint4* slot = reinterpret_cast<const uint4*>(smem + (size_t)((st & 1) * KW + kw) * SLOT) + lane;
+        const float sv = f16_bits_to_f32(scol[st * KW]);
+        h8_t B[8];
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
+        for (int t = 0; t < 8; ++t) B[t] = dequant8(w[t >> 2][t & 3], kc);
+        if constexpr (!kLast) load_w(min(st + 2, ns - 1), w);
+        // 32-row tiles in pairs (two independent accumulation chains), then their scale in fp32
 #pragma unroll
-            for (int t = 0; t < 4; ++t) A[mt][t] = __builtin_bit_cast(h8_t, slot[((4 * wm + mt) * 4 + t) * 64 + lane]);
-        float sv[4];
+        for (int mp = 0; mp < MT; mp += 2) {
+            constexpr int kPair = 2;
+            f16_t c[kPair];
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt) sv[nt] = f16_bits_to_f32(tsc[(64 * wn + 16 * nt + jn) * ngs + g]);
-        // column tiles in pairs: dequantise the pair's codes, then per m tile pair the 4 MFMA steps on 2 x 2 tiles
-        // (four independent chains) and their affine
+            for (int i = 0; i < kPair; ++i)
 #pragma unroll
-        for (int np = 0; np < 4; np += 2) {
-            h8_t B[2][4];
+                for (int e = 0; e < 16; ++e) c[i][e] = 0.f;
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int t = 0; t < 8; ++t)
 #pragma unroll
-                for (int t = 0; t < 4; ++t) B[j][t] = dequant8(w[np + j][t], kc);
-            if constexpr (!decltype(last)::value)
-                if (np == 2) load_w(min(g + 2, ngs - 1), w);
+                for (int i = 0; i < kPair; ++i)
+                    if (mp + i < MT)
+                        c[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            __builtin_bit_cast(h8_t, slot[((mp + i) * 8 + t) * 64]), B[t], c[i], 0, 0, 0);
 #pragma unroll
-            for (int mp = 0; mp < 4; mp += 2) {
-                f4_t c[2][2];
+            for (int i = 0; i < kPair; ++i)
+                if (mp + i < MT)
 #pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j)
-                            c[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mp + i][t], B[j][t],
-                                                                            t == 0 ? f4_t{0.f, 0.f, 0.f, 0.f} : c[i][j],
-                                                                            0, 0, 0);
-                // D[i][j]: row 4 (lane / 16) + e of the m tile, column lane % 16 of the tile: scale in fp32
-#pragma unroll
-                for (int i = 0; i < 2; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            acc[mp + i][np + j][e] = __builtin_fmaf(c[i][j][e], sv[np + j], acc[mp + i][np + j][e]);
-            }
+                    for (int e = 0; e < 16; ++e) acc[mp + i][e] = __builtin_fmaf(c[i][e], sv, acc[mp + i][e]);
         }
     };
-    // NG is even. Step 0 runs before the loop: the code loads above may be issued in any order, and a code register
-    // possibly in flight at the loop's first wait would make the compiler's waits in every iteration vmcnt(0); from
-    // step 1 on the load order is the loop's own. The last step, after the loop, issues no loads.
-    using more = std::integral_constant<bool, false>;
-    __builtin_assume(ngs >= 4);  // the loop runs at least once (the host checks)
-    step(0, 0, wa, more{});
-    for (int g = 1; g + 1 < ngs; g += 2) {
-        step(g, 1, wb, more{});
-        step(g + 1, 0, wa, more{});
+    // Step 0 runs before the loop: the code loads above may be issued in any order, and a code register possibly in
+    // flight at the loop's first wait would make the compiler's waits in every iteration vmcnt(0); from step 1 on
+    // the load order is the loop's own. The last step issues no loads. ns >= 2 (the host checks).
+    using yes = std::integral_constant<bool, true>;
+    using no = std::integral_constant<bool, false>;
+    step(0, wa, no{});
+    int st = 1;
+    for (; st + 2 < ns; st += 2) {
+        step(st, wb, no{});
+        step(st + 1, wa, no{});
     }
-    step(ngs - 1, 1, wb, std::integral_constant<bool, true>{});
+    if (st + 2 == ns) {
+        step(st, wb, no{});
+        step(st + 1, wa, yes{});
+    } else {
+        step(st, wb, yes{});
+    }
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (0 << 8));  // vmcnt(0) lgkmcnt(0): copies landed, ring reads done
     __builtin_amdgcn_s_barrier();                           // every wave has left the ring
     asm volatile("" ::: "memory");
 
-    // the wave's 64 x 64 tile through LDS ([64][65] fp32), then 16-byte row pieces: lane -> row 8 i + lane / 8,
-    // columns 8 (lane % 8) .. + 7
-    float* tb = reinterpret_cast<float*>(smem) + wave * (64 * 65);
+    // the waves' BM x 32 tiles through LDS ([BM][33] fp32), then 16-byte row pieces: K way kw writes the rows
+    // kw BM / KW .. of its columns (the ways' tiles added in order), lane -> row 16 i + lane / 4, columns
+    // 8 (lane % 4) .. + 7
+    float* tb = reinterpret_cast<float*>(smem) + wave * (BM * 33);
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+    for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) tb[(mt * 16 + 4 * sq + e) * 65 + 16 * nt + jn] = acc[mt][nt][e];
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave reads back only its own tile
-    const int m0 = mb + 64 * wm, n0 = nb + 64 * wn;
+        for (int e = 0; e < 16; ++e) tb[(32 * mt + 8 * (e >> 2) + 4 * hf + (e & 3)) * 33 + jn] = acc[mt][e];
+    if constexpr (KW == 1)
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the wave reads back only its own tile
+    else
+        __syncthreads();
+    const float* ot = reinterpret_cast<const float*>(smem) + cw * (BM * 33);
     if (splits > 1) Y = reinterpret_cast<float*>(Y) + (size_t)sp * M * ldy;  // this split's partial sums
     const bool vec_ok = (((uintptr_t)Y | (size_t)ldy * (ydt == RK_F32 ? 4 : 2)) & (ydt == RK_F32 ? 15 : 7)) == 0;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int r = 8 * i + (lane >> 3), cc = 8 * (lane & 7);
-        const int m = m0 + r, n = n0 + cc;
+    for (int i = 0; i < BM / KW / 16; ++i) {
+        const int r = kw * (BM / KW) + 16 * i + (lane >> 2), cc = 8 * (lane & 3);
+        const int m = mb + r, n = nb + 32 * cw + cc;
         if (m >= M || n >= N) continue;
-        const float* p = tb + r * 65 + cc;
+        float p[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            p[e] = ot[r * 33 + cc + e];
+#pragma unroll
+            for (int k = 1; k < KW; ++k) p[e] += ot[k * CW * (BM * 33) + r * 33 + cc + e];
+        }
         const size_t o = (size_t)m * ldy + n;
         if (n + 7 < N && vec_ok) {
             if (ydt == RK_F32) {
@@ -1156,9 +1169,9 @@ hipError_t launch_mm_prep(const void* X, int xdt, int ldx, const uint8_t* q, con
     float* xs = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + (size_t)Mp * K * 2);
     const dim3 pg((unsigned)(Mp / 16 * NG));  // one block per (m tile, group)
     if (xdt == RK_BF16)
-        hipLaunchKernelGGL((mm_xprep_kernel<true>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
+        hipLaunchKernelGGL((mm_xprep_kernel<true, false>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
     else
-        hipLaunchKernelGGL((mm_xprep_kernel<false>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
+        hipLaunchKernelGGL((mm_xprep_kernel<false, false>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
     const dim3 grid(((N + 127) / 128) * ((Mp + BM - 1) / BM));
     hipLaunchKernelGGL((mm_int4_prep_kernel<MT>), grid, dim3(512), mm_prep_lds_bytes<MT>(NG), st, Xp, xs, Mp, q, s, m,
                        Y, ydt, ldy, M, N, K);
@@ -1195,6 +1208,31 @@ __global__ __launch_bounds__(256) void mm_splitk_reduce4(const float* __restrict
 // sums follow the prepared X in the workspace and mm_splitk_reduce adds them in split order.
 size_t mm_wide_part_offset(int M, int K) { return (mm_prep_ws_bytes(M, K) + 255) / 256 * 256; }
 
+// Block shape of the wide-wave kernel: row blocks of equal height (3 or 4 tiles of 32 rows), and two K ways when one
+// round of a block per CU takes them all (measured, one K way -> two: 80 x 25088 x 2048 29.6 -> 21.2 us, 300 x 2048 x
+// 11008 45 -> 36; with more blocks two blocks per CU win: 512 x 25088 x 2048 74 against 89, 1024 x 2048 x 11008 70
+// against 79).
+struct WideShape {
+    int mt, kw;
+    long blocks;
+};
+inline WideShape wide_shape(int M, int N, int splits) {
+    const int t32 = (M + 31) / 32, rb = (t32 + 3) / 4, mt = std::max(3, (t32 + rb - 1) / rb);
+    const long blocks = (long)((N + kWideCols - 1) / kWideCols) * ((M + 32 * mt - 1) / (32 * mt)) * splits;
+    return {mt, blocks <= 256 ? 2 : 1, blocks};
+}
+
+template <int MT, int KW>
+hipError_t launch_mm_wide_cfg(const uint4* Xp, const float* xs, int Mp, const uint8_t* q, const uint16_t* s,
+                              const uint16_t* m, void* Y, int ydt, int ldy, int M, int N, int K, int splits,
+                              long blocks, hipStream_t st) {
+    int g_lo, ngs;
+    wide_split(K / 128, splits, splits - 1, g_lo, ngs);  // the last split has the most groups
+    hipLaunchKernelGGL((mm_int4_wide_kernel<MT, KW>), dim3((unsigned)blocks), dim3(256 * KW),
+                       (mm_wide_lds_bytes<MT, KW>(ngs)), st, Xp, xs, Mp, q, s, m, Y, ydt, ldy, M, N, K, splits);
+    return hipGetLastError();
+}
+
 hipError_t launch_mm_wide(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
                           void* Y, int ydt, int ldy, int M, int N, int K, int splits, void* ws, hipStream_t st) {
     const int NG = K / 128, Mp = (M + 15) / 16 * 16;
@@ -1202,28 +1240,26 @@ hipError_t launch_mm_wide(const void* X, int xdt, int ldx, const uint8_t* q, con
     float* xs = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + (size_t)Mp * K * 2);
     const dim3 pg((unsigned)(Mp / 16 * NG));  // one block per (m tile, group)
     if (xdt == RK_BF16)
-        hipLaunchKernelGGL((mm_xprep_kernel<true>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
+        hipLaunchKernelGGL((mm_xprep_kernel<true, true>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
     else
-        hipLaunchKernelGGL((mm_xprep_kernel<false>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
-    const int tiles = ((N + 127) / 128) * ((Mp + 127) / 128);
-    int g_lo, ngs;
-    wide_split(NG, splits, splits - 1, g_lo, ngs);  // the last split has the most groups
-    const size_t lds = mm_wide_lds_bytes(ngs);
-    if (splits == 1) {
-        hipLaunchKernelGGL(mm_int4_wide_kernel, dim3(tiles), dim3(256), lds, st, Xp, xs, Mp, q, s, m, Y, ydt, ldy,
-                           M, N, K, 1);
-    } else {
-        float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + mm_wide_part_offset(M, K));
-        hipLaunchKernelGGL(mm_int4_wide_kernel, dim3(tiles * splits), dim3(256), lds, st, Xp, xs, Mp, q, s, m,
-                           (void*)part, (int)RK_F32, N, M, N, K, splits);
-        const size_t mn = (size_t)M * N;
-        if (N % 4 == 0)
-            hipLaunchKernelGGL(mm_splitk_reduce4, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, part,
-                               splits, Y, ydt, ldy, M, N);
-        else
-            hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits,
-                               Y, ydt, ldy, M, N);
-    }
+        hipLaunchKernelGGL((mm_xprep_kernel<false, true>), pg, dim3(256), 0, st, X, ldx, M, Mp, K, Xp, xs);
+    const WideShape sh = wide_shape(M, N, splits);
+    float* part = reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + mm_wide_part_offset(M, K));
+    void* out = splits == 1 ? Y : (void*)part;
+    const int odt = splits == 1 ? ydt : (int)RK_F32, ldo = splits == 1 ? ldy : N;
+#define RK_WIDE(MT, KW) \
+    launch_mm_wide_cfg<MT, KW>(Xp, xs, Mp, q, s, m, out, odt, ldo, M, N, K, splits, sh.blocks, st)
+    const hipError_t e = sh.mt == 3 ? (sh.kw == 2 ? RK_WIDE(3, 2) : RK_WIDE(3, 1))
+                                    : (sh.kw == 2 ? RK_WIDE(4, 2) : RK_WIDE(4, 1));
+#undef RK_WIDE
+    if (e != hipSuccess || splits == 1) return e;
+    const size_t mn = (size_t)M * N;
+    if (N % 4 == 0)
+        hipLaunchKernelGGL(mm_splitk_reduce4, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
+                           Y, ydt, ldy, M, N);
+    else
+        hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits, Y,
+                           ydt, ldy, M, N);
     return hipGetLastError();
 }
 
@@ -1306,8 +1342,8 @@ constexpr size_t kLdsMax = 160 * 1024;
 
 // Kernel choice for one shape. With a caller's workspace (rk_mm_int4_g128_ws) and enough 128-column blocks to give
 // most CUs one (cfg 3 / 4 / 5: the prepared-X kernel with 128 / 64 / 48-row blocks; its workspace holds the prepared
-// X; cfg 7 ahead of them for M > 64 when K / 128 is even and >= 4: the wide-wave kernel, two blocks per CU, split
-// over K when its tiles are few). Otherwise 128 x 128 tiles (cfg 1) when that still gives every CU a block, else 64 x 64 tiles (cfg 2), split
+// X; cfg 7 ahead of them for M > 64 when K / 128 is even and >= 4: the wide-wave kernel, split over K when its tiles are
+// few). Otherwise 128 x 128 tiles (cfg 1) when that still gives every CU a block, else 64 x 64 tiles (cfg 2), split
 // over K when a workspace or the fixed scratch is allowed and the tiles alone leave CUs idle (each split keeps >= 4
 // groups); cfg 0 is the register-staged kernel, for K too long to stage one block's scales in LDS.
 struct MmPlan {
@@ -1332,24 +1368,30 @@ MmPlan mm_stream_plan(int M, int N, int K, int mode) {
 
 MmPlan mm_plan(int M, int N, int K, int mode);
 
-// The wide-wave plan (cfg 7) for M > 64 and an even group count >= 4: splits over K (whole pairs of groups, >= 4
-// groups and <= kWideMaxGroups each) only when the 128 x 128 tiles alone leave the chip's two-blocks-per-CU slots
-// mostly idle, M >= 256 and K / 128 > 16; used when tiles x splits reaches kPrepMinBlocks. The workspace holds the prepared X, the partial
-// sums when split, and at least what the tile plan that unaligned scale / min arrays fall back to needs.
-constexpr long kWideSlots = 512;  // two blocks per CU on 256 CUs
+// The wide-wave plan (cfg 7) for M > 64 and an even group count >= 4. From kWideMinTiles tiles of 128 x 128 on, one
+// block per tile (measured against the 64 x 64 tiles: 149 tiles, 100 x 19000 x 2048, 24 us against 36; 144 tiles, 700 x
+// 3072 x 2048, 26 against 33; 128 tiles, 512 x 4096 x 2048, 25 against 23). Fewer tiles are split over K (whole pairs
+// of groups, >= 4 and <= kWideMaxGroups groups each) for M > 128 and K / 128 > 16: the fp32 partial sums (S x M x N)
+// and the reduce launch cost more than they give for short K or few rows (512 x 3072 x 2048 34 us against 24, 128 x
+// 2048 x 11008 32 against 26). Below 64 tiles the splits fill one block of two K ways per CU (200 x 2048 x 11008 29 us,
+// 41 on the 64 x 64 tiles; 300 x 2048 x 11008 36 against 48 with twice the splits); from 64 on two blocks per CU (512 x
+// 2048 x 11008 45 us against 43 for half the splits in two K ways). The workspace holds the prepared X, the partial sums
+// when split, and at least what the tile plan that unaligned scale / min arrays fall back to needs.
+constexpr long kWideMinTiles = 136;
 MmPlan mm_wide_plan(int M, int N, int K) {
     const int NG = K / 128, P = NG / 2;
     const long Mp = (M + 15) / 16 * 16;
     const long tiles = (long)((N + 127) / 128) * ((Mp + 127) / 128);
     const int smin = (P + kWideMaxGroups / 2 - 1) / (kWideMaxGroups / 2);
-    if (tiles >= kPrepMinBlocks && smin > 1) return {-1, 0, 0};  // enough tiles: no split just to fit the tables
-    // few tiles: the split's fp32 partial sums (S x M x N) and the reduce launch paid off only for long K at large M
-    // (measured: 512 x 2048 x 11008 58 us against 75 on the tile plan; 512 x 3072 x 2048 34 against 24,
-    // 128 x 2048 x 11008 32 against 26)
-    if (tiles < kPrepMinBlocks && (M < 256 || NG <= 16)) return {-1, 0, 0};
+    const bool few = tiles < kWideMinTiles;
+    if (!few && smin > 1) return {-1, 0, 0};  // enough tiles: no split just to fit the tables
+    if (few && (M <= 128 || NG <= 16)) return {-1, 0, 0};
     int S = smin;
-    if (tiles < kPrepMinBlocks) S = std::max<long>(smin, std::min<long>((kWideSlots + tiles / 2) / tiles, P / 2));
-    if (S > P / 2 || tiles * S < kPrepMinBlocks) return {-1, 0, 0};
+    if (few) {
+        const long fill = tiles < 64 ? 256 / tiles : (512 + tiles / 2) / tiles;
+        S = std::max<long>(smin, std::min<long>(fill, P / 2));
+    }
+    if (S > P / 2 || tiles * S < kWideMinTiles) return {-1, 0, 0};
     size_t ws = S > 1 ? mm_wide_part_offset(M, K) + (size_t)S * M * N * sizeof(float) : mm_prep_ws_bytes(M, K);
     ws = std::max(ws, mm_plan(M, N, K, kMmScratch).ws);
     return {7, S, ws};
