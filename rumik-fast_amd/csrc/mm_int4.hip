@@ -226,15 +226,12 @@ struct MmStage {
 // code rows of the next two steps in registers and, during step g, convert step g + 1 into the other LDS stage
 // (X -> fp16 fragments, codes -> exact fp16). One barrier per step; the two roles run on every SIMD at once, so
 // the staging conversions overlap the MFMAs instead of following them.
-// Split K (splits > 1): block (tile, split) covers groups [split NG / splits, (split + 1) NG / splits) and writes
-// its fp32 sums to part[split][M][N] for mm_splitk_reduce; with splits == 1 the block writes Y directly.
 // BF16: activations are bf16 (else fp16), a template parameter so the staging has no per-chunk dtype branches
 template <int WM, int WN, bool BF16>
 __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict__ X, int ldx,
                                                           const uint8_t* __restrict__ q, const uint16_t* __restrict__ sc,
                                                           const uint16_t* __restrict__ mn, void* __restrict__ Y,
-                                                          int ydt, int ldy, int M, int N, int K,
-                                                          float* __restrict__ part, int splits) {
+                                                          int ydt, int ldy, int M, int N, int K) {
     constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
     constexpr int XCH = BM * 16 / 256;  // 16-byte X chunks per staging thread per step (row r, 8-column block c)
     constexpr int WCH = BN * 4 / 256;   // 16-byte code chunks per staging thread per step (row n, quarter s)
@@ -251,15 +248,13 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
     // contiguous range, walked row block fastest: the row blocks sharing one code tile run together on one L2
     const int G = gridDim.x, L = blockIdx.x, GY = (M + BM - 1) / BM;
     const int Lv = (G % 8 == 0) ? (L % 8) * (G / 8) + L / 8 : L;
-    const int split = Lv % splits, tile = Lv / splits;
-    const int mb = (tile % GY) * BM, nb = (tile / GY) * BN;
-    const int NGT = K >> 7;                                                   // groups of a row
-    const int g0 = split * NGT / splits, NG = (split + 1) * NGT / splits - g0;  // this block's groups
+    const int mb = (Lv % GY) * BM, nb = (Lv / GY) * BN;
+    const int NG = K >> 7;
     uint32_t* smw = reinterpret_cast<uint32_t*>(stg + 2);  // [BN][NG]: scale | min << 16 of the block's rows
 
     for (int i = tid; i < BN * NG; i += 512) {
-        const int n = min(nb + i / NG, N - 1), g = g0 + i % NG;
-        smw[i] = (uint32_t)sc[(size_t)n * NGT + g] | ((uint32_t)mn[(size_t)n * NGT + g] << 16);
+        const int n = min(nb + i / NG, N - 1), g = i % NG;
+        smw[i] = (uint32_t)sc[(size_t)n * NG + g] | ((uint32_t)mn[(size_t)n * NG + g] << 16);
     }
     // staging slots: X chunk i -> row r = idx / 16, 8-column block c = idx % 16 (a row's 256 bytes in 16
     // consecutive lanes); code chunk i -> row r = idx % 16 + 16 (idx / 64),
@@ -274,13 +269,13 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
             const int idx = sid + 256 * i, r = idx >> 4, c = idx & 15;
             const int m = min(mb + r, M - 1);
             xr[i] = *reinterpret_cast<const u4_t*>(reinterpret_cast<const uint16_t*>(X) + (size_t)m * ldx +
-                                                   128 * (g0 + g) + 8 * c);
+                                                   128 * g + 8 * c);
         }
 #pragma unroll
         for (int i = 0; i < WCH; ++i) {
             const int idx = sid + 256 * i, r = (idx & 15) | ((idx >> 6) << 4), qq = (idx >> 4) & 3;
             const int n = min(nb + r, N - 1);
-            wr[i] = *reinterpret_cast<const u4_t*>(q + (size_t)n * (size_t)(K >> 1) + 64 * (g0 + g) + 16 * qq);
+            wr[i] = *reinterpret_cast<const u4_t*>(q + (size_t)n * (size_t)(K >> 1) + 64 * g + 16 * qq);
         }
     };
     auto store = [&](const Regs& R, Stage& st) {
@@ -388,12 +383,222 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
             for (int e = 0; e < 4; ++e) {
                 const int m = mb + (wm * WM + mt) * 16 + 4 * (lane >> 4) + e;
                 if (m >= M) continue;
-                if (splits == 1)
-                    store_act(Y, ydt, (size_t)m * ldy + n, acc[mt][nt][e]);
-                else
-                    part[((size_t)split * M + m) * N + n] = acc[mt][nt][e];
+                store_act(Y, ydt, (size_t)m * ldy + n, acc[mt][nt][e]);
             }
         }
+}
+
+// ---------------------------------------------------------------------------------------------- 64 x 64 tiles
+// mm_int4_tile64_kernel: a block of W waves owns a (16 MT) x (16 NT) tile of Y and a range of K groups; the waves
+// split the groups (wave w takes every W-th one) and each computes the whole tile over its own, so the K loop has
+// no barrier and no shared staging: eight independent streams per CU, two per SIMD, whose loads, conversions and
+// MFMAs overlap as they fall. A group's X rows come by global_load_lds into the wave's own LDS buffer (16-byte
+// chunks of 256-byte rows, 64 lanes = 4 rows; chunk c of row r sits at position c ^ (r % 16), so the fragment reads
+// of 16 rows touch 16 distinct bank groups), its codes into registers; both are issued for the wave's next group as
+// soon as this group's fragments have been read. The block's scales and mins are read once into LDS (gathered per
+// group and wave, two bytes a lane, they cost 1.2 us per step). Row sums over the group are MFMAs of the fragments
+// against ones; the min terms are added four groups at a time as fp32 MFMAs (K = 4). The waves' sums meet in LDS
+// after the loop (in wave order).
+// The L2 delivers ~50 B/clk to every CU (31 TB/s over the chip, measured), so re-reading X per column block (20 KB
+// per 64 x 64 x 128 step) is not what bounds it; the conversions and MFMAs of two waves per SIMD are (2.2 us per
+// 64 x 64 x 128 step and wave).
+// Split K (splits > 1): block (split, tile) covers groups [split NG / splits, (split + 1) NG / splits) and writes
+// its fp32 sums to part[split][M][N] for mm_splitk_reduce; with splits == 1 the block writes Y directly. The splits
+// are the slowest index, so an XCD's L2 holds a few K ranges of X instead of all of it.
+// Requires ldx and K <= kTile64MaxStride (32-bit offsets within a tile); the host checks both.
+constexpr int kTile64MaxStride = 1 << 25;
+constexpr size_t kTile64MaxLds = 160 * 1024;
+constexpr int kTile64MaxGroups = 384;  // of one block: four waves' buffers of four m tiles and the table are 160 KiB
+
+// the waves' X buffers (reused for their sums) and the scale / min table of ngb groups
+inline size_t tile64_lds_bytes(int MT, int NT, int W, int ngb) {
+    return (size_t)W * MT * 4096 + (size_t)16 * NT * 4 * ngb;
+}
+
+template <int MT, int NT, int W, bool BF16>
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void mm_int4_tile64_kernel(const uint16_t* __restrict__ X, int ldx, const uint8_t* __restrict__ q,
+                           const uint16_t* __restrict__ sc, const uint16_t* __restrict__ mn, void* __restrict__ Y,
+                           int ydt, int ldy, int M, int N, int K, float* __restrict__ part, int splits) {
+    constexpr int BM = 16 * MT, BN = 16 * NT;
+    extern __shared__ __align__(16) uint8_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int jn = lane & 15, sq = lane >> 4;
+    // 1-D grid: workgroups go round-robin to the 8 XCDs, so virtual id (L % 8) * (G / 8) + L / 8 gives each XCD a
+    // contiguous range, walked row block fastest: the row blocks sharing one code tile run together on one L2
+    const int G = gridDim.x, L = blockIdx.x, GY = (M + BM - 1) / BM, T = G / splits;
+    const int Lv = (G % 8 == 0) ? (L % 8) * (G / 8) + L / 8 : L;
+    const int split = Lv / T, tile = Lv - split * T;
+    const int mb = (tile % GY) * BM, nb = (tile / GY) * BN;
+    const int NG = K >> 7, KB = K >> 1;
+    const int g0 = (int)((long)split * NG / splits), g1 = (int)((long)(split + 1) * NG / splits);
+    uint4* xb = reinterpret_cast<uint4*>(smem) + wave * (MT * 256);  // this wave's X rows: [BM][16 chunks]
+
+    // byte offsets of this lane's X chunks within an m tile (copy i of a tile: rows 4 i + lane / 16), for whole tiles
+    // and for the one tile that reaches past M (rows past M repeat row M - 1)
+    const int mlast = (M - 1 - mb) >> 4;  // the block's last m tile with rows (>= 0)
+    uint32_t xo[4], xe[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = 4 * i + sq, c = jn ^ r;
+        xo[i] = (uint32_t)r * (uint32_t)(2 * ldx) + 16 * c;
+        xe[i] = (uint32_t)min(r, M - 1 - mb - 16 * mlast) * (uint32_t)(2 * ldx) + 16 * c;
+    }
+    uint32_t wo[NT];  // this lane's code bytes: column 16 nt + jn (clamped), bytes 16 sq .. + 15 of each group
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) wo[nt] = (uint32_t)(min(nb + 16 * nt + jn, N - 1) - nb) * (uint32_t)KB + 16 * sq;
+    const uint8_t* qb = q + (size_t)nb * KB;
+    const uint8_t* xbase = reinterpret_cast<const uint8_t*>(X) + (size_t)mb * ldx * 2;
+
+    auto load_w = [&](int g, u4_t (&w)[NT]) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) w[nt] = *reinterpret_cast<const u4_t*>(qb + (size_t)64 * g + wo[nt]);
+    };
+    auto issue_x = [&](int g) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int mc = min(mt, mlast);  // m tiles past M repeat the last one; they are never stored
+            const uint8_t* src = xbase + (size_t)mc * 32 * ldx + (size_t)256 * g;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint4*>(src + (mc == mlast ? xe[i] : xo[i])),
+                                                 xb + (mt * 4 + i) * 64, 16, 0, 0);
+        }
+    };
+
+    f4_t acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
+    // row sums and mins of up to four groups as K = 4 operands: lane (row or column l % 16, group l / 16)
+    float xa[MT], mv[NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) xa[mt] = 0.f;
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) mv[nt] = 0.f;
+    auto add_min = [&]() {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[mt], mv[nt], acc[mt][nt], 0, 0, 0);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) xa[mt] = 0.f;
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) mv[nt] = 0.f;
+    };
+    const DqConsts kc = {opaque(0x000F000Fu), opaque(0x00F000F0u), opaque(0x64006400u)};
+    const h8_t ones = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f,
+                       (_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f};
+    int g = g0 + wave, idx = 0;
+    u4_t wn[NT];
+    if (g < g1) {
+        load_w(g, wn);
+        issue_x(g);
+    }
+    const int ngb = g1 - g0;
+    uint32_t* tab = reinterpret_cast<uint32_t*>(smem + (size_t)W * MT * 4096);  // [ngb][BN] scale | min << 16
+    for (int i = tid; i < BN * ngb; i += 64 * W) {
+        const int c = i / ngb, gi = i - c * ngb;
+        const size_t o = (size_t)min(nb + c, N - 1) * NG + g0 + gi;
+        tab[gi * BN + c] = (uint32_t)sc[o] | ((uint32_t)mn[o] << 16);
+    }
+    __syncthreads();
+    for (; g < g1; g += W) {
+        // this group's loads and copies have landed (they are the only ones in flight)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0)
+        asm volatile("" ::: "memory");
+        h8_t A[MT][4];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+                A[mt][t] = __builtin_bit_cast(h8_t, xb[mt * 256 + jn * 16 + ((4 * sq + t) ^ jn)]);
+        u4_t wq[NT];
+        uint32_t sm[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            wq[nt] = wn[nt];
+            sm[nt] = tab[(g - g0) * BN + 16 * nt + jn];
+        }
+        // the fragments are in registers: the wave's buffer may be refilled
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4) | (0 << 8));  // lgkmcnt(0)
+        asm volatile("" ::: "memory");
+        if (g + W < g1) {
+            load_w(g + W, wn);
+            issue_x(g + W);
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            f4_t xs = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                A[mt][t] = afrag(__builtin_bit_cast(u4_t, A[mt][t]), BF16 ? RK_BF16 : RK_F16);
+                xs = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, A[mt][t], xs, 0, 0, 0);  // D[.][j] = sum of row j
+            }
+            xa[mt] = sq == (idx & 3) ? xs[0] : xa[mt];
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            const uint32_t smn = sm[nt];
+            const float scl = f16_bits_to_f32((uint16_t)smn);
+            mv[nt] = sq == (idx & 3) ? f16_bits_to_f32((uint16_t)(smn >> 16)) : mv[nt];
+            f4_t c[MT];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const h8_t B = dequant8(wq[nt][t], kc);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    c[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mt][t], B, t == 0 ? f4_t{0.f, 0.f, 0.f, 0.f} : c[mt],
+                                                                  0, 0, 0);
+            }
+            // D[i][j]: row 4 (lane / 16) + e of the m tile, column lane % 16 of the column tile: scale in fp32
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[mt][nt][e] = __builtin_fmaf(c[mt][e], scl, acc[mt][nt][e]);
+        }
+        if ((idx & 3) == 3) add_min();
+        ++idx;
+    }
+    if (idx & 3) add_min();
+
+    // the waves' sums through LDS (each in its own buffer, whose copies have all been read), added in wave order
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));  // vmcnt(0): the last (surplus) copies have landed
+    asm volatile("" ::: "memory");
+    f4_t* rb = reinterpret_cast<f4_t*>(xb);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) rb[(mt * NT + nt) * 64 + lane] = acc[mt][nt];
+    __syncthreads();
+    for (int it = tid; it < MT * NT * 64; it += 64 * W) {
+        f4_t u[W];
+#pragma unroll
+        for (int w = 0; w < W; ++w) u[w] = reinterpret_cast<const f4_t*>(smem)[w * (MT * 256) + it];
+        f4_t v = u[0];
+#pragma unroll
+        for (int w = 1; w < W; ++w)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += u[w][e];
+        const int l = it & 63, nt = (it >> 6) % NT, mt = it / (64 * NT);
+        const int n = nb + 16 * nt + (l & 15);
+        if (n >= N) continue;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = mb + 16 * mt + 4 * (l >> 4) + e;
+            if (m >= M) continue;
+            if (splits == 1)
+                store_act(Y, ydt, (size_t)m * ldy + n, v[e]);
+            else
+                part[((size_t)split * M + m) * N + n] = v[e];
+        }
+    }
 }
 
 // ---------------------------------------------------------------------------------------------- prepared-X kernel
@@ -1178,13 +1383,22 @@ hipError_t launch_mm_prep(const void* X, int xdt, int ldx, const uint8_t* q, con
     return hipGetLastError();
 }
 
-// Y[m, n] = sum over splits of part[split][m][n] (fixed order), in Y's dtype
+// Y[m, n] = sum over splits of part[split][m][n] (fixed order), in Y's dtype. Bound by latency (a few MB over the whole
+// chip): eight splits' loads are in flight at a time (one after the other, 8 splits of 60 x 2048 took 4.0 us).
+constexpr int kReduceBatch = 8;
 __global__ __launch_bounds__(256) void mm_splitk_reduce(const float* __restrict__ part, int splits,
                                                         void* __restrict__ Y, int ydt, int ldy, int M, int N) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, MN = (size_t)M * N;
     if (i >= MN) return;
     float v = 0.f;
-    for (int k = 0; k < splits; ++k) v += part[k * MN + i];
+    for (int k = 0; k < splits; k += kReduceBatch) {
+        float p[kReduceBatch];
+#pragma unroll
+        for (int j = 0; j < kReduceBatch; ++j) p[j] = part[min(k + j, splits - 1) * MN + i];
+#pragma unroll
+        for (int j = 0; j < kReduceBatch; ++j)
+            if (k + j < splits) v += p[j];
+    }
     store_act(Y, ydt, (i / N) * ldy + i % N, v);
 }
 
@@ -1194,10 +1408,17 @@ __global__ __launch_bounds__(256) void mm_splitk_reduce4(const float* __restrict
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4, MN = (size_t)M * N;
     if (i >= MN) return;
     f4_t v = {0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < splits; ++k) {
-        const f4_t p = *reinterpret_cast<const f4_t*>(part + k * MN + i);
+    for (int k = 0; k < splits; k += kReduceBatch) {
+        f4_t p[kReduceBatch];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += p[e];
+        for (int j = 0; j < kReduceBatch; ++j)
+            p[j] = *reinterpret_cast<const f4_t*>(part + min(k + j, splits - 1) * MN + i);
+#pragma unroll
+        for (int j = 0; j < kReduceBatch; ++j)
+            if (k + j < splits) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += p[j][e];
+            }
     }
     const size_t o = (i / N) * ldy + i % N;
 #pragma unroll
@@ -1298,6 +1519,66 @@ hipError_t launch_mm_stream(const void* X, int xdt, int ldx, const uint8_t* q, c
     return launch_mm_stream_mt<3>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, st);
 }
 
+// Y (or, split, the partial sums and their ordered sum) of the 64 x 64 tiles: row blocks of at most four m tiles of
+// equal height
+template <int MT, int NT, int W>
+hipError_t launch_mm_tile64_cfg(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s,
+                                const uint16_t* m, void* Y, int ydt, int ldy, int M, int N, int K, float* part,
+                                int splits, hipStream_t st) {
+    const dim3 grid((unsigned)(((N + 16 * NT - 1) / (16 * NT)) * ((M + 16 * MT - 1) / (16 * MT)) * splits));
+    const size_t lds = tile64_lds_bytes(MT, NT, W, (K / 128 + splits - 1) / splits);
+    const uint16_t* x = static_cast<const uint16_t*>(X);
+    if (xdt == RK_BF16)
+        hipLaunchKernelGGL((mm_int4_tile64_kernel<MT, NT, W, true>), grid, dim3(64 * W), lds, st, x, ldx, q, s, m, Y,
+                           ydt, ldy, M, N, K, part, splits);
+    else
+        hipLaunchKernelGGL((mm_int4_tile64_kernel<MT, NT, W, false>), grid, dim3(64 * W), lds, st, x, ldx, q, s, m, Y,
+                           ydt, ldy, M, N, K, part, splits);
+    return hipGetLastError();
+}
+
+template <int MT>
+hipError_t launch_mm_tile64_mt(int nt, int w, const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s,
+                               const uint16_t* m, void* Y, int ydt, int ldy, int M, int N, int K, float* part,
+                               int splits, hipStream_t st) {
+    if (w == 8 && nt == 1)
+        return launch_mm_tile64_cfg<MT, 1, 8>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st);
+    if (w == 8 && nt == 2)
+        return launch_mm_tile64_cfg<MT, 2, 8>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st);
+    if (w == 8) return launch_mm_tile64_cfg<MT, 4, 8>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st);
+    return launch_mm_tile64_cfg<MT, 4, 4>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st);
+}
+
+hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
+                            void* Y, int ydt, int ldy, int M, int N, int K, float* part, int splits, hipStream_t st) {
+    const int t16 = (M + 15) / 16, rb = (t16 + 3) / 4, mt = (t16 + rb - 1) / rb, ngb = (K / 128 + splits - 1) / splits;
+    const long tiles = (long)((N + 63) / 64) * rb;
+    // the narrowest columns that still give every CU at most one block; otherwise 64 columns, by eight waves while one
+    // round takes all blocks and every wave has a group, else by four and two blocks per CU. Measured with 16 / 32 / 64 columns: 69 x 2048
+    // x 2048 6.6 / 7.7 / 10.5 us, 200 x 2048 x 2048 14.2 / 9.7 / 12.8, 512 x 2048 x 2048 26 / 17.3 / 13.1; eight / four
+    // waves: 512 x 2048 x 2048 13.1 / 15.4, 512 x 3072 x 2048 23.9 / 20.0.
+    const long b64 = tiles * splits;
+    const int nt = 4 * b64 <= 256 ? 1 : 2 * b64 <= 256 ? 2 : 4;
+    const bool w8 = nt < 4 || (b64 <= 256 && ngb >= 8);
+    const int w = w8 && tile64_lds_bytes(mt, nt, 8, ngb) <= kTile64MaxLds ? 8 : 4;
+    hipError_t e;
+    switch (mt) {
+        case 1: e = launch_mm_tile64_mt<1>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
+        case 2: e = launch_mm_tile64_mt<2>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
+        case 3: e = launch_mm_tile64_mt<3>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
+        default: e = launch_mm_tile64_mt<4>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
+    }
+    if (e != hipSuccess || splits == 1) return e;
+    const size_t mn = (size_t)M * N;
+    if (N % 4 == 0)
+        hipLaunchKernelGGL(mm_splitk_reduce4, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
+                           Y, ydt, ldy, M, N);
+    else
+        hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits, Y,
+                           ydt, ldy, M, N);
+    return hipGetLastError();
+}
+
 template <int WM, int WN>
 size_t mm_lds_bytes(int ng) {  // ng: groups of one block
     constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
@@ -1306,21 +1587,16 @@ size_t mm_lds_bytes(int ng) {  // ng: groups of one block
 
 template <int WM, int WN>
 hipError_t launch_mm_lds(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
-                         void* Y, int ydt, int ldy, int M, int N, int K, float* part, int splits, hipStream_t st) {
+                         void* Y, int ydt, int ldy, int M, int N, int K, hipStream_t st) {
     constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
-    const size_t lds = mm_lds_bytes<WM, WN>((K / 128 + splits - 1) / splits);
-    dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits);
+    const size_t lds = mm_lds_bytes<WM, WN>(K / 128);
+    dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM));
     if (xdt == RK_BF16)
         hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, true>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt, ldy,
-                           M, N, K, part, splits);
+                           M, N, K);
     else
         hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, false>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt,
-                           ldy, M, N, K, part, splits);
-    if (splits > 1) {
-        const size_t mn = (size_t)M * N;
-        hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits, Y,
-                           ydt, ldy, M, N);
-    }
+                           ldy, M, N, K);
     return hipGetLastError();
 }
 
@@ -1345,7 +1621,7 @@ constexpr size_t kLdsMax = 160 * 1024;
 // X; cfg 7 ahead of them for M > 64 when K / 128 is even and >= 4: the wide-wave kernel, split over K when its tiles are
 // few). Otherwise 128 x 128 tiles (cfg 1) when that still gives every CU a block, else 64 x 64 tiles (cfg 2), split
 // over K when a workspace or the fixed scratch is allowed and the tiles alone leave CUs idle (each split keeps >= 4
-// groups); cfg 0 is the register-staged kernel, for K too long to stage one block's scales in LDS.
+// groups); cfg 0 is the register-staged kernel, for K too long to hold one block's scales in LDS.
 struct MmPlan {
     int cfg, splits;
     size_t ws;  // workspace bytes: fp32 partials (cfg 2 with splits > 1) or the prepared X (cfg 3 - 5)
@@ -1417,9 +1693,13 @@ MmPlan mm_plan(int M, int N, int K, int mode) {
     if (M > 64 && big >= 256 && mm_lds_bytes<4, 4>(NG) <= kLdsMax) return {1, 1, 0};
     const long small = (long)((N + 63) / 64) * ((M + 63) / 64);
     int splits = 1;
-    if (allow_ws && small < 256) splits = (int)std::max(1L, std::min((256 + small - 1) / small, (long)(NG / 4)));
-    while (allow_ws && mm_lds_bytes<2, 2>((NG + splits - 1) / splits) > kLdsMax && splits < NG) ++splits;
-    if (mm_lds_bytes<2, 2>((NG + splits - 1) / splits) > kLdsMax) return {0, 1, 0};
+    // K <= 2048 takes a few steps of eight waves: no split. Up to 7680 only as many splits as fill the chip with
+    // 16-column blocks (their partial sums are the fewest: 48 x 2048 x 5120 10.8 us against 12.8 for eight splits of 64
+    // columns); longer K as many as fill it with 64-column blocks. A split keeps >= 4 groups.
+    if (allow_ws && small < 256 && NG > 16)
+        splits = (int)std::max(1L, std::min(NG <= 60 ? (63 + small) / small : 256 / small, (long)(NG / 4)));
+    while (allow_ws && (NG + splits - 1) / splits > kTile64MaxGroups && splits < NG) ++splits;
+    if ((NG + splits - 1) / splits > kTile64MaxGroups) return {0, 1, 0};
     return {2, splits, splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0};
 }
 
@@ -1436,11 +1716,13 @@ int mm_check(const void* X, int x_dtype, int ldx, const uint8_t* q, const uint16
 int mm_run(const MmPlan& p, const void* X, int x_dtype, int ldx, const uint8_t* q, const uint16_t* scale,
            const uint16_t* min, void* Y, int y_dtype, int ldy, int M, int N, int K, void* ws, hipStream_t s) {
     hipError_t e;
-    if (p.cfg == 1)
-        e = launch_mm_lds<4, 4>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, nullptr, 1, s);
+    if (p.cfg == 2 && (ldx > kTile64MaxStride || K > kTile64MaxStride))  // offsets past 32 bits: the register-staged kernel
+        e = launch_mm<2, 2>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, s);
+    else if (p.cfg == 1)
+        e = launch_mm_lds<4, 4>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, s);
     else if (p.cfg == 2)
-        e = launch_mm_lds<2, 2>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, static_cast<float*>(ws),
-                                p.splits, s);
+        e = launch_mm_tile64(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, static_cast<float*>(ws),
+                             p.splits, s);
     else if (p.cfg == 3)
         e = launch_mm_prep<8>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, ws, s);
     else if (p.cfg == 4)
