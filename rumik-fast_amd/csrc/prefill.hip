@@ -11,20 +11,14 @@
 // prefill_attn on the matrix cores (v_mfma_f32_16x16x32_f16; operand layouts: A[i][k] in lane i + 16 (k / 8),
 // element k % 8; B[k][j] in lane j + 16 (k / 8); D[i][j] in lane j + 16 (i / 4), element i % 4). Block = (KV head
 // g, a share of its query heads, tile of 16 queries); wave r = the share's head r. Per key block of 32 slots the
-// block stages K [32 x 128] and V transposed [128 x 32] in LDS once for its heads; each wave computes S^T = K Q^T (2 x 4
-// MFMAs), the causal mask and an online softmax in log2 units (lazy running max, see the key loop), and accumulates
-// O^T += V^T P^T (8 MFMAs, fp32; P in fp16, the reference's tensor-core PV in 16-bit). The products are taken
-// transposed, over keys ordered so that a lane's 8 scores of one query are the 8 consecutive keys of its P^T fragment:
-// P never leaves the lane's registers, and m, l and the rescale are one value per lane.
-// The launch time is the longest query tile's key loop, whose steps are bound by the waves' own LDS traffic and VALU
-// work (one or two waves per SIMD), so the loop keeps the per-score instruction count down: the max is reduced across
-// lanes only when a ballot says some score exceeds its query's running max by more than 8 (log2 units, a factor of
-// 256), O is rescaled only then, the sums stay per lane until the loop ends, and the causal mask is applied only on
-// blocks that reach past the tile's first query. Blocks start with the longest tiles, so that where a prompt has more
-// blocks than fit the chip at once the short ones fill in behind them.
-// us per launch, 16 query heads, against P through LDS, tiles in ascending order and a merge of one group at a time:
-// NKV 4: T = 69 6.7 -> 5.6, 200 9.1 -> 7.7, 512 13.9 -> 11.9, 1024 33.2 -> 24.8 (28.6 in ascending order), 2000
-// 92.9 -> 72.8; T = 1024 with NKV 8 38.0 -> 24.9, NKV 16 44.3 -> 31.7, NKV 2 38.9 -> 35.5.
+// block stages K [32 x 128] and V transposed [128 x 32] in LDS once for its heads; each wave computes S = Q K^T (2 x 4
+// MFMAs), the causal mask and an online softmax in log2 units (lazy running max, see the key loop), stores P (fp16,
+// the reference's tensor-core PV in 16-bit) to its LDS tile in the A layout and accumulates O += P V (8 MFMAs, fp32).
+// The launch time is the longest query tile's key loop, whose steps are bound by the waves' VALU work (one or two
+// waves per SIMD), so the loop keeps the per-score instruction count down: the row max is reduced across lanes only
+// when a ballot says some score exceeds its row's running max by more than 8 (log2 units, a factor of 256), O is
+// rescaled only then, the row sums stay per lane until the loop ends, and the causal mask is applied only on blocks
+// that reach past the tile's first query.
 #include "common.h"
 
 #include <initializer_list>
@@ -349,6 +343,22 @@ __global__ __launch_bounds__(kPostPart) void post_rows_vec_kernel(const uint16_t
     }
 }
 
+// all-reduce over the 16 lanes of a DPP row (row_ror 8, 4, 2, 1)
+RK_DEV float row16_max(float v) {
+    v = fmaxf(v, dpp<0x128>(v));
+    v = fmaxf(v, dpp<0x124>(v));
+    v = fmaxf(v, dpp<0x122>(v));
+    v = fmaxf(v, dpp<0x121>(v));
+    return v;
+}
+RK_DEV float row16_sum(float v) {
+    v += dpp<0x128>(v);
+    v += dpp<0x124>(v);
+    v += dpp<0x122>(v);
+    v += dpp<0x121>(v);
+    return v;
+}
+
 // grid (NKV * (NH / NKV) / REP, ceil(T / 16)), 64 * REP * KS threads: block x = (KV head g, share z) computes query
 // heads g (NH / NKV) + z REP .. + REP - 1. q: [T, NH * 128] fp16 (RoPE applied); kc / vc: the layer's cache
 // [NKV, S, 128] fp16 holding slots 0 .. p0 + T - 1; o: [T, NH * 128] fp16. Query t attends slots 0 .. p0 + t.
@@ -379,8 +389,6 @@ constexpr int kChunksPerKB = kKB * kHD / 8;  // 512
 constexpr int kVtRow = kKB + 8;     // QUAD: halves per Vt row (80 bytes)
 constexpr int kVtBlk = kHD * kVtRow;  // QUAD: halves per key block of Vt (the CHUNK form uses kHD * kKB of them)
 
-// row of Ks that holds key j of its block: MFMA row i of half hf is key 8 (i / 4) + 4 hf + i % 4, at Ks row 16 hf + i
-RK_DEV int ks_row(int j) { return 16 * ((j >> 2) & 1) + 4 * (j >> 3) + (j & 3); }
 // column of key j in transposed row d
 RK_DEV int vt_col(int d, int j) { return (j + 8 * ((d >> 3) & 3)) & (kKB - 1); }
 // offset in halves of key j of dim row d of Vt key block b (j a multiple of 4 for QUAD, of 8 for CHUNK)
@@ -419,7 +427,7 @@ RK_DEV void kv_store(const KVChunks<CH>& c, uint16_t (*Ks)[kKB][kHD + kKsPad], u
             const int qd = threadIdx.x + g * blockDim.x, kb = qd / (kChunksPerKB / 4), qq = qd % (kChunksPerKB / 4);
             const int k4 = 4 * (qq / (kHD / 8)), d8 = (qq % (kHD / 8)) * 8;
 #pragma unroll
-            for (int u = 0; u < 4; ++u) *reinterpret_cast<u4_t*>(&Ks[kb][ks_row(k4) + u][d8]) = c.k[4 * g + u];
+            for (int u = 0; u < 4; ++u) *reinterpret_cast<u4_t*>(&Ks[kb][k4 + u][d8]) = c.k[4 * g + u];
 #pragma unroll
             for (int w = 0; w < 4; ++w) {  // dims d8 + 2w (low halves) and d8 + 2w + 1 (high halves) of the 4 keys
                 const uint32_t v0 = c.v[4 * g][w], v1 = c.v[4 * g + 1][w], v2 = c.v[4 * g + 2][w], v3 = c.v[4 * g + 3][w];
@@ -434,7 +442,7 @@ RK_DEV void kv_store(const KVChunks<CH>& c, uint16_t (*Ks)[kKB][kHD + kKsPad], u
         for (int u = 0; u < CH; ++u) {
             const int e = threadIdx.x + u * blockDim.x, kb = e / kChunksPerKB, ep = e % kChunksPerKB;
             const int kj = ep / (kHD / 8), d8 = (ep % (kHD / 8)) * 8;
-            *reinterpret_cast<u4_t*>(&Ks[kb][ks_row(kj)][d8]) = c.k[u];
+            *reinterpret_cast<u4_t*>(&Ks[kb][kj][d8]) = c.k[u];
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
                 Vt[vt_off<false>(kb, d8 + 2 * w, kj)] = (uint16_t)c.v[u][w];
@@ -444,15 +452,14 @@ RK_DEV void kv_store(const KVChunks<CH>& c, uint16_t (*Ks)[kKB][kHD + kKsPad], u
     }
 }
 
-// dynamic LDS of prefill_attn_kernel<REP, KS>: the staging (KS key blocks of K and transposed V), reused after the key
-// loop for the merge (a partial result of 128 x 16 fp32 plus m / l per query for each wave)
-constexpr int kMergeWave = 64 * 32 + 2 * kQT;  // floats per wave
-constexpr size_t attn_stage_bytes(int KS) {
-    return (size_t)KS * kKB * (kHD + kKsPad) * 2 + (size_t)KS * kVtBlk * 2;
+// dynamic LDS of prefill_attn_kernel<REP, KS>: the staging (KS key blocks of K and transposed V, one P tile per
+// wave), reused after the key loop for the merge (REP partial results of 16 x 128 fp32 plus m / l per row)
+constexpr size_t attn_stage_bytes(int REP, int KS) {
+    return (size_t)KS * kKB * (kHD + kKsPad) * 2 + (size_t)KS * kVtBlk * 2 + (size_t)REP * KS * kQT * kKB * 2;
 }
-constexpr size_t attn_merge_bytes(int REP, int KS) { return KS > 1 ? (size_t)REP * KS * kMergeWave * 4 : 0; }
+constexpr size_t attn_merge_bytes(int REP) { return (size_t)REP * (64 * 32 + 2 * kQT) * 4; }
 constexpr size_t attn_lds_bytes(int REP, int KS) {
-    return attn_stage_bytes(KS) > attn_merge_bytes(REP, KS) ? attn_stage_bytes(KS) : attn_merge_bytes(REP, KS);
+    return attn_stage_bytes(REP, KS) > attn_merge_bytes(REP) ? attn_stage_bytes(REP, KS) : attn_merge_bytes(REP);
 }
 
 template <int REP, int KS>
@@ -466,14 +473,16 @@ __global__ __launch_bounds__(64 * REP * KS) __attribute__((amdgpu_waves_per_eu(1
     auto Ks = reinterpret_cast<uint16_t(*)[kKB][kHD + kKsPad]>(lds);
     constexpr bool QUAD = CH % 4 == 0;
     uint16_t* Vt = reinterpret_cast<uint16_t*>(lds + (size_t)KS * kKB * (kHD + kKsPad) * 2);
+    uint16_t* Ps = reinterpret_cast<uint16_t*>(lds + (size_t)KS * kKB * (kHD + kKsPad) * 2 + (size_t)KS * kVtBlk * 2);
     const int shares = NH / NKV / REP;
-    const int g = blockIdx.x / shares, q0 = (gridDim.y - 1 - blockIdx.y) * kQT;  // the longest tiles first
+    const int g = blockIdx.x / shares, q0 = blockIdx.y * kQT;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r = w % REP, ks = w / REP;
     const int h = g * (NH / NKV) + (blockIdx.x % shares) * REP + r;
-    const int li = lane & 15, lq = lane >> 4;  // fragments: row or column li, k-group lq; this lane's query q0 + li
+    const int li = lane & 15, lq = lane >> 4;  // A / B fragment: row or column li, k-group lq
     const float sl2 = scale * 1.44269504088896341f;  // scores in log2 units: P = 2^(s sl2 - m)
     const int ldq = NH * kHD;
+    uint16_t* P = Ps + w * kQT * kKB;
     // Q fragments of this wave's head: query q0 + li, dims 32c + 8 lq .. + 8
     h8_t Qf[4];
     {
@@ -488,8 +497,12 @@ __global__ __launch_bounds__(64 * REP * KS) __attribute__((amdgpu_waves_per_eu(1
     f4_t O[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) O[c] = f4_t{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    const int qpos = p0 + q0 + li;
+    float m[4], l[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        m[e] = -INFINITY;
+        l[e] = 0.f;
+    }
     const uint16_t* kg = kc + (size_t)g * S * kHD;
     const uint16_t* vg = vc + (size_t)g * S * kHD;
     const int last = p0 + min(q0 + kQT, T) - 1;  // the last slot any query of the tile sees
@@ -511,8 +524,7 @@ __global__ __launch_bounds__(64 * REP * KS) __attribute__((amdgpu_waves_per_eu(1
     kv_load<CH>(kg, vg, kb0 + ((st) + 2) * KS, last, cur);  /* two steps ahead (clamped past the end) */ \
     if (kb0 + (st) * KS + ks < kb1) {  /* wave-uniform: this group's key block of the step exists */ \
         const int j0 = (kb0 + (st) * KS + ks) * kKB; \
-        /* S^T = K Q^T: d[hf][e] is key j0 + 8 lq + 4 hf + e of query li, so a lane's 8 scores are 8 consecutive keys */ \
-        /* of one query: its fragment of P^T for the second product, with no exchange between lanes */ \
+        /* S = Q K^T for keys j0 + 16 hf + li (D layout: row 4 lq + e, key li) */ \
         /* all 8 K fragments are read before the first MFMA (the reads' latencies overlap instead of adding up) */ \
         h8_t Bk[2][4]; \
 _Pragma("unroll") \
@@ -527,52 +539,68 @@ _Pragma("unroll") \
         for (int hf = 0; hf < 2; ++hf) { \
             f4_t d = {0.f, 0.f, 0.f, 0.f}; \
 _Pragma("unroll") \
-            for (int c = 0; c < 4; ++c) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bk[hf][c], Qf[c], d, 0, 0, 0); \
+            for (int c = 0; c < 4; ++c) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(Qf[c], Bk[hf][c], d, 0, 0, 0); \
             Sd[hf] = d; \
         } \
         /* scores in log2 units (scale * log2 e folded in); the causal mask only on blocks that reach past the */ \
-        /* tile's first query (wave-uniform). Lazy running max: a query's m moves only when one of the block's */ \
+        /* tile's first query (wave-uniform). Lazy running max: a row's m moves only when one of the block's */ \
         /* scores exceeds it by more than kLazyMax, so P = 2^(s - m) <= 2^kLazyMax (fp16 holds it at the same */ \
-        /* relative precision); a lane-local compare and one ballot decide, and only then are the query's maxima */ \
-        /* reduced over its four lanes and O rescaled. l holds per-lane partial sums (reduced after the key loop). */ \
+        /* relative precision); a lane-local compare and one ballot decide, and only then are the row maxima */ \
+        /* reduced and O rescaled. l holds per-lane partial sums (reduced across the row after the key loop). */ \
         const bool diag = j0 + kKB - 1 > p0 + q0; \
-        float sc[8]; \
+        float sc0[4], sc1[4]; \
+        bool big = false; \
 _Pragma("unroll") \
-        for (int e = 0; e < 8; ++e) { \
-            sc[e] = Sd[e >> 2][e & 3] * sl2; \
-            if (diag && j0 + 8 * lq + e > qpos) sc[e] = -INFINITY; \
+        for (int e = 0; e < 4; ++e) { \
+            sc0[e] = Sd[0][e] * sl2; \
+            sc1[e] = Sd[1][e] * sl2; \
+            if (diag) { \
+                const int qpos = p0 + q0 + 4 * lq + e; \
+                if (j0 + li > qpos) sc0[e] = -INFINITY; \
+                if (j0 + 16 + li > qpos) sc1[e] = -INFINITY; \
+            } \
+            big = big || fmaxf(sc0[e], sc1[e]) > m[e] + kLazyMax; /* never for a masked score */ \
         } \
-        float mb = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7]))); \
-        if (__any(mb > m + kLazyMax)) { /* never for a masked score */ \
-            mb = fmaxf(mb, __shfl_xor(mb, 16)); \
-            mb = fmaxf(mb, __shfl_xor(mb, 32)); \
-            if (mb > m + kLazyMax) { /* the same in the query's four lanes */ \
-                const float alpha = __builtin_amdgcn_exp2f(m - mb);  /* m = -inf: 0 (O and l are still 0) */ \
-                m = mb; \
-                l *= alpha; \
+        float alpha[4] = {1.f, 1.f, 1.f, 1.f}; \
+        const bool moved = __any(big); \
+        if (moved) { \
 _Pragma("unroll") \
-                for (int c = 0; c < 8; ++c) \
-_Pragma("unroll") \
-                    for (int e = 0; e < 4; ++e) O[c][e] *= alpha; \
+            for (int e = 0; e < 4; ++e) { \
+                const float mb = row16_max(fmaxf(sc0[e], sc1[e])); \
+                if (mb > m[e] + kLazyMax) { \
+                    alpha[e] = __builtin_amdgcn_exp2f(m[e] - mb);  /* m = -inf: 0 (O and l are still 0) */ \
+                    m[e] = mb; \
+                } \
             } \
         } \
-        h8_t Pf; \
-        float ls = 0.f; \
 _Pragma("unroll") \
-        for (int e = 0; e < 8; ++e) { \
-            Pf[e] = (_Float16)(m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sc[e] - m)); \
-            ls += (float)Pf[e]; \
+        for (int e = 0; e < 4; ++e) { \
+            const float p0v = m[e] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sc0[e] - m[e]); \
+            const float p1v = m[e] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(sc1[e] - m[e]); \
+            const _Float16 h0 = (_Float16)p0v, h1 = (_Float16)p1v; \
+            l[e] = l[e] * alpha[e] + ((float)h0 + (float)h1); \
+            P[(4 * lq + e) * kKB + li] = __builtin_bit_cast(uint16_t, h0); \
+            P[(4 * lq + e) * kKB + 16 + li] = __builtin_bit_cast(uint16_t, h1); \
         } \
-        l += ls; \
-        /* O^T += V^T P^T: A = Vt[dim 16 c + li][keys 8 lq .. + 8], B = P^T[keys 8 lq .. + 8][query li] */ \
+        if (moved) { \
+_Pragma("unroll") \
+            for (int c = 0; c < 8; ++c) \
+_Pragma("unroll") \
+                for (int e = 0; e < 4; ++e) O[c][e] *= alpha[e]; \
+        } \
+        __builtin_amdgcn_wave_barrier(); \
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); \
+        /* O += P V: A = P[query li][keys 8 lq .. + 8], B = Vt[dim 16 c + li][keys 8 lq .. + 8] */ \
+        const h8_t A = __builtin_bit_cast(h8_t, *reinterpret_cast<const uint4*>(&P[li * kKB + 8 * lq])); \
         h8_t Bv[8]; \
 _Pragma("unroll") \
         for (int c = 0; c < 8; ++c) \
             Bv[c] = __builtin_bit_cast(h8_t, *reinterpret_cast<const uint4*>(Vt + vt_off<QUAD>(ks, 16 * c + li, 8 * lq))); \
-        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0); \
+        __builtin_amdgcn_sched_group_barrier(0x100, 9, 0); \
         __builtin_amdgcn_sched_group_barrier(0x008, 8, 0); \
 _Pragma("unroll") \
-        for (int c = 0; c < 8; ++c) O[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(Bv[c], Pf, O[c], 0, 0, 0); \
+        for (int c = 0; c < 8; ++c) O[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, Bv[c], O[c], 0, 0, 0); \
+        __builtin_amdgcn_wave_barrier();  /* P is rewritten in the next step only after these reads */ \
     } \
     do {} while (0)
     // both steps of an iteration run unconditionally (a step past the tile's last key block stages clamped slots and
@@ -583,63 +611,52 @@ _Pragma("unroll") \
         RK_ATTN_STEP(st + 1, kb);
     }
 #undef RK_ATTN_STEP
-    l += __shfl_xor(l, 16);  // the query's partial sums across its four lanes
-    l += __shfl_xor(l, 32);
-    // merge the KS partials of each head in one exchange: every wave leaves (O, m, l) in LDS (lane-major O, m / l per
-    // query), then wave ks of a head sums dims 16 c .. + 16 for its 8 / KS values of c over the groups, in group order
-    constexpr int CO = 8 / KS;  // dim blocks of 16 a wave finishes
-    f4_t R[CO];
-    float lt = l;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) l[e] = row16_sum(l[e]);  // the row's partial sums across its 16 lanes
+    // merge the KS partials of each head into group 0, one group at a time, in group order: (m, l, O) of group k
+    // through LDS (lane-major O, m / l per row), then m' = max, l' = l a + l_k b, O' = O a + O_k b
     if constexpr (KS > 1) {
-        float* mo = reinterpret_cast<float*>(lds) + (size_t)r * KS * kMergeWave;
-        __syncthreads();  // the staging is no longer read
-        float* mine = mo + ks * kMergeWave;
+        float* mo = reinterpret_cast<float*>(lds) + (size_t)r * (64 * 32 + 2 * kQT);
+        for (int k = 1; k < KS; ++k) {
+            __syncthreads();  // the staging (or the previous round's values) is no longer read
+            if (ks == k) {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) *reinterpret_cast<f4_t*>(mine + (c * 64 + lane) * 4) = O[c];
-        if (lq == 0) {
-            mine[64 * 32 + li] = m;
-            mine[64 * 32 + kQT + li] = l;
-        }
-        __syncthreads();
-        float mk[KS], mn = -INFINITY;
+                for (int c = 0; c < 8; ++c)
 #pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            mk[k] = mo[k * kMergeWave + 64 * 32 + li];
-            mn = fmaxf(mn, mk[k]);
-        }
-        lt = 0.f;
+                    for (int e = 0; e < 4; ++e) mo[(c * 4 + e) * 64 + lane] = O[c][e];
+                if (li == 0) {
 #pragma unroll
-        for (int c = 0; c < CO; ++c) R[c] = f4_t{0.f, 0.f, 0.f, 0.f};
+                    for (int e = 0; e < 4; ++e) {
+                        mo[64 * 32 + 4 * lq + e] = m[e];
+                        mo[64 * 32 + kQT + 4 * lq + e] = l[e];
+                    }
+                }
+            }
+            __syncthreads();
+            if (ks == 0) {
 #pragma unroll
-        for (int k = 0; k < KS; ++k) {
-            const float a = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mk[k] - mn);  // m in log2 units
-            lt += mo[k * kMergeWave + 64 * 32 + kQT + li] * a;
+                for (int e = 0; e < 4; ++e) {
+                    const float mk = mo[64 * 32 + 4 * lq + e], lk = mo[64 * 32 + kQT + 4 * lq + e];
+                    const float mn = fmaxf(m[e], mk);
+                    const float a = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m[e] - mn);  // m in log2 units
+                    const float b = mn == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mk - mn);
+                    l[e] = l[e] * a + lk * b;
+                    m[e] = mn;
 #pragma unroll
-            for (int c = 0; c < CO; ++c)
-                R[c] += *reinterpret_cast<const f4_t*>(mo + k * kMergeWave + ((ks * CO + c) * 64 + lane) * 4) * a;
-        }
-    } else {
-#pragma unroll
-        for (int c = 0; c < CO; ++c) R[c] = O[c];
-    }
-    const int t = q0 + li;
-    if (t >= T) return;
-    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
-    uint16_t* orow = o + (size_t)t * ldq + h * kHD + 16 * ks * CO + 4 * lq;
-    const bool wide = ((uintptr_t)o & 7) == 0;  // q, kc and vc are checked to be aligned, o may lie anywhere
-#pragma unroll
-    for (int c = 0; c < CO; ++c) {
-        const h4_t hv = {(_Float16)(R[c][0] * inv), (_Float16)(R[c][1] * inv), (_Float16)(R[c][2] * inv),
-                         (_Float16)(R[c][3] * inv)};
-        if (wide) {
-            *reinterpret_cast<h4_t*>(orow + 16 * c) = hv;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const _Float16 v = hv[e];  // a value: bit_cast of a vector's element itself reads element 0
-                orow[16 * c + e] = __builtin_bit_cast(uint16_t, v);
+                    for (int c = 0; c < 8; ++c) O[c][e] = O[c][e] * a + mo[(c * 4 + e) * 64 + lane] * b;
+                }
             }
         }
+    }
+    if (ks != 0) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int t = q0 + 4 * lq + e;
+        if (t >= T) continue;
+        const float inv = l[e] > 0.f ? 1.0f / l[e] : 0.f;
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            o[(size_t)t * ldq + h * kHD + 16 * c + li] = __builtin_bit_cast(uint16_t, (_Float16)(O[c][e] * inv));
     }
 }
 
@@ -743,8 +760,7 @@ extern "C" int rk_prefill_attn(const void* q, const void* kc, const void* vc, vo
                        dim3(64 * (HPB) * (K)), attn_lds_bytes(HPB, K), st, (const uint16_t*)q, (const uint16_t*)kc,   \
                        (const uint16_t*)vc, (uint16_t*)o, T, p0, NH, NKV, S, scale)
     // the launch time is the longest query tile's key loop (p0 + T keys): past 384 keys four key groups per block
-    // (two waves per SIMD) beat two (T = 512: 13.9 against 14.5 us, with P still through LDS; at T = 16 .. 256 two
-    // are faster)
+    // (two waves per SIMD) beat two (T = 512: 13.9 against 14.5 us; at T = 16 .. 256 two are faster)
     const bool long_keys = p0 + T > 384;
     switch (rep) {
         case 1: RK_ATTN(1, kAttnKS); break;
