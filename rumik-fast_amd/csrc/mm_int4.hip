@@ -29,10 +29,13 @@ struct DqConsts {
     uint32_t lo_mask, hi_mask, magic;
 };
 
-RK_DEV h8_t dequant8(uint32_t w, const DqConsts& k) {
-    const h2_t m1024 = {(_Float16)-1024.f, (_Float16)-1024.f};
+// 8 codes less BIAS (0 or 8) as fp16, exact: 1024 + code and 64 + code are fp16 values, their difference from
+// 1024 + BIAS or 64 + BIAS a small whole number
+template <int BIAS>
+RK_DEV h8_t dequant8_less(uint32_t w, const DqConsts& k) {
+    const h2_t m1024 = {(_Float16)(-1024.f - BIAS), (_Float16)(-1024.f - BIAS)};
     const h2_t s16 = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const h2_t m64 = {(_Float16)-64.f, (_Float16)-64.f};
+    const h2_t m64 = {(_Float16)(-64.f - BIAS), (_Float16)(-64.f - BIAS)};
     const uint32_t b = w >> 8;
     const h2_t p0 = as_h2((w & k.lo_mask) | k.magic) + m1024;
     const h2_t p1 = as_h2((w & k.hi_mask) | k.magic) * s16 + m64;
@@ -43,6 +46,16 @@ RK_DEV h8_t dequant8(uint32_t w, const DqConsts& k) {
     r[4] = p2.x; r[5] = p2.y; r[6] = p3.x; r[7] = p3.y;
     return r;
 }
+
+RK_DEV h8_t dequant8(uint32_t w, const DqConsts& k) { return dequant8_less<0>(w, k); }
+
+// Centred codes, for the kernels that sum the min terms apart from the scaled products: code * scale + min =
+// (code - 8) * scale + centred_min. A quantised group lies around zero (min near -7.5 scale), so with raw codes the two
+// sums are large and cancel wherever a row's activations have a mean; centred, both are small, in the same number of
+// instructions. Error of fp32 outputs against 64 bits, activations of mean 1: 512 x 3072 x 2048 (64 x 64 tiles)
+// 5.8e-7 -> 7.6e-8, 300 x 5000 x 8192 (wide, split) 2.0e-6 -> 1.8e-7; sums taken group by group have 3.4e-7 / 3.9e-7.
+RK_DEV h8_t dequant8_centred(uint32_t w, const DqConsts& k) { return dequant8_less<8>(w, k); }
+RK_DEV float centred_min(float min, float scale) { return __builtin_fmaf(8.f, scale, min); }
 
 // 8 consecutive activations (one 16-byte load) -> A fragment (x0,x4,x1,x5,x2,x6,x3,x7) as fp16
 RK_DEV h8_t afrag(u4_t d, int xdt) {
@@ -397,8 +410,8 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
 // of 16 rows touch 16 distinct bank groups), its codes into registers; both are issued for the wave's next group as
 // soon as this group's fragments have been read. The block's scales and mins are read once into LDS (gathered per
 // group and wave, two bytes a lane, they cost 1.2 us per step). Row sums over the group are MFMAs of the fragments
-// against ones; the min terms are added four groups at a time as fp32 MFMAs (K = 4). The waves' sums meet in LDS
-// after the loop (in wave order).
+// against ones; the (centred) min terms are added four groups at a time as fp32 MFMAs (K = 4). The waves' sums meet
+// in LDS after the loop (in wave order).
 // The L2 delivers ~50 B/clk to every CU (31 TB/s over the chip, measured), so re-reading X per column block (20 KB
 // per 64 x 64 x 128 step) is not what bounds it; the conversions and MFMAs of two waves per SIMD are (2.2 us per
 // 64 x 64 x 128 step and wave).
@@ -473,21 +486,24 @@ void mm_int4_tile64_kernel(const uint16_t* __restrict__ X, int ldx, const uint8_
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f4_t{0.f, 0.f, 0.f, 0.f};
     // row sums and mins of up to four groups as K = 4 operands: lane (row or column l % 16, group l / 16)
-    float xa[MT], mv[NT];
+    // (the mins as table words, scale | min << 16, until they are added)
+    float xa[MT];
+    uint32_t mv[NT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) xa[mt] = 0.f;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) mv[nt] = 0.f;
+    for (int nt = 0; nt < NT; ++nt) mv[nt] = 0u;
     auto add_min = [&]() {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int nt = 0; nt < NT; ++nt) {
+            const float v = centred_min(f16_bits_to_f32((uint16_t)(mv[nt] >> 16)), f16_bits_to_f32((uint16_t)mv[nt]));
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[mt], mv[nt], acc[mt][nt], 0, 0, 0);
+            for (int mt = 0; mt < MT; ++mt)
+                acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[mt], v, acc[mt][nt], 0, 0, 0);
+            mv[nt] = 0u;
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) xa[mt] = 0.f;
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) mv[nt] = 0.f;
     };
     const DqConsts kc = {opaque(0x000F000Fu), opaque(0x00F000F0u), opaque(0x64006400u)};
     const h8_t ones = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f,
@@ -546,11 +562,11 @@ void mm_int4_tile64_kernel(const uint16_t* __restrict__ X, int ldx, const uint8_
         for (int nt = 0; nt < NT; ++nt) {
             const uint32_t smn = sm[nt];
             const float scl = f16_bits_to_f32((uint16_t)smn);
-            mv[nt] = sq == (idx & 3) ? f16_bits_to_f32((uint16_t)(smn >> 16)) : mv[nt];
+            mv[nt] = sq == (idx & 3) ? smn : mv[nt];
             f4_t c[MT];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const h8_t B = dequant8(wq[nt][t], kc);
+                const h8_t B = dequant8_centred(wq[nt][t], kc);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
                     c[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[mt][t], B, t == 0 ? f4_t{0.f, 0.f, 0.f, 0.f} : c[mt],
@@ -837,8 +853,8 @@ RK_PREP_INST(8)
 //     per lane and step;
 //   * codes go straight into registers, two steps ahead; X copies go into a two-step LDS ring with
 //     global_load_lds, one barrier per step;
-//   * the min term sum_g xs[m][g] min[n][g] is each accumulator's starting value, computed on the matrix cores in
-//     fp32 (v_mfma_f32_32x32x2f32, two groups per instruction) while the first copies land, from row sums copied
+//   * the (centred) min term sum_g xs[m][g] min[n][g] is each accumulator's starting value, computed on the matrix
+//     cores in fp32 (v_mfma_f32_32x32x2f32, two groups per instruction) while the first copies land, from row sums copied
 //     into the ring slot that step 0 leaves free; the per-step affine is one FMA per output (scale).
 // The ring slot of step s + 1 is filled after the barrier of step s, which every wave passes only once it has
 // left step s - 1 (the slot's previous step).
@@ -978,7 +994,8 @@ __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))
     const uint16_t* mcol = tmn + (32 * cw + jn) * ngs + kw;
     for (int p = 0; p < ns; p += 2) {
         const int st = p + hf;
-        const float mv = st < ns ? f16_bits_to_f32(mcol[st * KW]) : 0.f;
+        const float mv =
+            st < ns ? centred_min(f16_bits_to_f32(mcol[st * KW]), f16_bits_to_f32(scol[st * KW])) : 0.f;
         float xa[MT];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) xa[mt] = st < ns ? xsl[(st * KW + kw) * BM + 32 * mt + jn] : 0.f;
@@ -999,7 +1016,7 @@ __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))
         const float sv = f16_bits_to_f32(scol[st * KW]);
         h8_t B[8];
 #pragma unroll
-        for (int t = 0; t < 8; ++t) B[t] = dequant8(w[t >> 2][t & 3], kc);
+        for (int t = 0; t < 8; ++t) B[t] = dequant8_centred(w[t >> 2][t & 3], kc);
         if constexpr (!kLast) load_w(min(st + 2, ns - 1), w);
         // 32-row tiles in pairs (two independent accumulation chains), then their scale in fp32
 #pragma unroll
