@@ -239,12 +239,15 @@ struct MmStage {
 // code rows of the next two steps in registers and, during step g, convert step g + 1 into the other LDS stage
 // (X -> fp16 fragments, codes -> exact fp16). One barrier per step; the two roles run on every SIMD at once, so
 // the staging conversions overlap the MFMAs instead of following them.
+// Split K (splits > 1): block (tile, split) covers groups [split NG / splits, (split + 1) NG / splits) and writes
+// its fp32 sums to part[split][M][N] for mm_splitk_reduce; with splits == 1 the block writes Y directly.
 // BF16: activations are bf16 (else fp16), a template parameter so the staging has no per-chunk dtype branches
 template <int WM, int WN, bool BF16>
 __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict__ X, int ldx,
                                                           const uint8_t* __restrict__ q, const uint16_t* __restrict__ sc,
                                                           const uint16_t* __restrict__ mn, void* __restrict__ Y,
-                                                          int ydt, int ldy, int M, int N, int K) {
+                                                          int ydt, int ldy, int M, int N, int K,
+                                                          float* __restrict__ part, int splits) {
     constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
     constexpr int XCH = BM * 16 / 256;  // 16-byte X chunks per staging thread per step (row r, 8-column block c)
     constexpr int WCH = BN * 4 / 256;   // 16-byte code chunks per staging thread per step (row n, quarter s)
@@ -261,13 +264,15 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
     // contiguous range, walked row block fastest: the row blocks sharing one code tile run together on one L2
     const int G = gridDim.x, L = blockIdx.x, GY = (M + BM - 1) / BM;
     const int Lv = (G % 8 == 0) ? (L % 8) * (G / 8) + L / 8 : L;
-    const int mb = (Lv % GY) * BM, nb = (Lv / GY) * BN;
-    const int NG = K >> 7;
+    const int split = Lv % splits, tile = Lv / splits;
+    const int mb = (tile % GY) * BM, nb = (tile / GY) * BN;
+    const int NGT = K >> 7;  // groups of a row; this block's are g0 .. g0 + NG - 1
+    const int g0 = (int)((long)split * NGT / splits), NG = (int)((long)(split + 1) * NGT / splits) - g0;
     uint32_t* smw = reinterpret_cast<uint32_t*>(stg + 2);  // [BN][NG]: scale | min << 16 of the block's rows
 
     for (int i = tid; i < BN * NG; i += 512) {
-        const int n = min(nb + i / NG, N - 1), g = i % NG;
-        smw[i] = (uint32_t)sc[(size_t)n * NG + g] | ((uint32_t)mn[(size_t)n * NG + g] << 16);
+        const int n = min(nb + i / NG, N - 1), g = g0 + i % NG;
+        smw[i] = (uint32_t)sc[(size_t)n * NGT + g] | ((uint32_t)mn[(size_t)n * NGT + g] << 16);
     }
     // staging slots: X chunk i -> row r = idx / 16, 8-column block c = idx % 16 (a row's 256 bytes in 16
     // consecutive lanes); code chunk i -> row r = idx % 16 + 16 (idx / 64),
@@ -282,13 +287,13 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
             const int idx = sid + 256 * i, r = idx >> 4, c = idx & 15;
             const int m = min(mb + r, M - 1);
             xr[i] = *reinterpret_cast<const u4_t*>(reinterpret_cast<const uint16_t*>(X) + (size_t)m * ldx +
-                                                   128 * g + 8 * c);
+                                                   128 * (size_t)(g0 + g) + 8 * c);
         }
 #pragma unroll
         for (int i = 0; i < WCH; ++i) {
             const int idx = sid + 256 * i, r = (idx & 15) | ((idx >> 6) << 4), qq = (idx >> 4) & 3;
             const int n = min(nb + r, N - 1);
-            wr[i] = *reinterpret_cast<const u4_t*>(q + (size_t)n * (size_t)(K >> 1) + 64 * g + 16 * qq);
+            wr[i] = *reinterpret_cast<const u4_t*>(q + (size_t)n * (size_t)(K >> 1) + 64 * (size_t)(g0 + g) + 16 * qq);
         }
     };
     auto store = [&](const Regs& R, Stage& st) {
@@ -396,7 +401,10 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
             for (int e = 0; e < 4; ++e) {
                 const int m = mb + (wm * WM + mt) * 16 + 4 * (lane >> 4) + e;
                 if (m >= M) continue;
-                store_act(Y, ydt, (size_t)m * ldy + n, acc[mt][nt][e]);
+                if (splits == 1)
+                    store_act(Y, ydt, (size_t)m * ldy + n, acc[mt][nt][e]);
+                else
+                    part[((size_t)split * M + m) * N + n] = acc[mt][nt][e];
             }
         }
 }
@@ -418,7 +426,7 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
 // Split K (splits > 1): block (split, tile) covers groups [split NG / splits, (split + 1) NG / splits) and writes
 // its fp32 sums to part[split][M][N] for mm_splitk_reduce; with splits == 1 the block writes Y directly. The splits
 // are the slowest index, so an XCD's L2 holds a few K ranges of X instead of all of it.
-// Requires ldx and K <= kTile64MaxStride (32-bit offsets within a tile); the host checks both.
+// Requires ldx and K <= kTile64MaxStride (32-bit offsets within a tile); mm_run checks both.
 constexpr int kTile64MaxStride = 1 << 25;
 constexpr size_t kTile64MaxLds = 160 * 1024;
 constexpr int kTile64MaxGroups = 384;  // of one block: four waves' buffers of four m tiles and the table are 160 KiB
@@ -1460,6 +1468,18 @@ inline WideShape wide_shape(int M, int N, int splits) {
     return {mt, blocks <= 256 ? 2 : 1, blocks};
 }
 
+hipError_t launch_splitk_reduce(const float* part, int splits, void* Y, int ydt, int ldy, int M, int N,
+                                hipStream_t st) {
+    const size_t mn = (size_t)M * N;
+    if (N % 4 == 0)
+        hipLaunchKernelGGL(mm_splitk_reduce4, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
+                           Y, ydt, ldy, M, N);
+    else
+        hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits, Y,
+                           ydt, ldy, M, N);
+    return hipGetLastError();
+}
+
 template <int MT, int KW>
 hipError_t launch_mm_wide_cfg(const uint4* Xp, const float* xs, int Mp, const uint8_t* q, const uint16_t* s,
                               const uint16_t* m, void* Y, int ydt, int ldy, int M, int N, int K, int splits,
@@ -1491,14 +1511,7 @@ hipError_t launch_mm_wide(const void* X, int xdt, int ldx, const uint8_t* q, con
                                     : (sh.kw == 2 ? RK_WIDE(4, 2) : RK_WIDE(4, 1));
 #undef RK_WIDE
     if (e != hipSuccess || splits == 1) return e;
-    const size_t mn = (size_t)M * N;
-    if (N % 4 == 0)
-        hipLaunchKernelGGL(mm_splitk_reduce4, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
-                           Y, ydt, ldy, M, N);
-    else
-        hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits, Y,
-                           ydt, ldy, M, N);
-    return hipGetLastError();
+    return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
 }
 
 template <int MT, int D>
@@ -1586,14 +1599,7 @@ hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, c
         default: e = launch_mm_tile64_mt<4>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
     }
     if (e != hipSuccess || splits == 1) return e;
-    const size_t mn = (size_t)M * N;
-    if (N % 4 == 0)
-        hipLaunchKernelGGL(mm_splitk_reduce4, dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0, st, part, splits,
-                           Y, ydt, ldy, M, N);
-    else
-        hipLaunchKernelGGL(mm_splitk_reduce, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st, part, splits, Y,
-                           ydt, ldy, M, N);
-    return hipGetLastError();
+    return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
 }
 
 template <int WM, int WN>
@@ -1604,17 +1610,19 @@ size_t mm_lds_bytes(int ng) {  // ng: groups of one block
 
 template <int WM, int WN>
 hipError_t launch_mm_lds(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
-                         void* Y, int ydt, int ldy, int M, int N, int K, hipStream_t st) {
+                         void* Y, int ydt, int ldy, int M, int N, int K, float* part, int splits, hipStream_t st) {
     constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
-    const size_t lds = mm_lds_bytes<WM, WN>(K / 128);
-    dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM));
+    const size_t lds = mm_lds_bytes<WM, WN>((K / 128 + splits - 1) / splits);
+    dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits);
     if (xdt == RK_BF16)
         hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, true>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt, ldy,
-                           M, N, K);
+                           M, N, K, part, splits);
     else
         hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, false>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt,
-                           ldy, M, N, K);
-    return hipGetLastError();
+                           ldy, M, N, K, part, splits);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || splits == 1) return e;
+    return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
 }
 
 template <int WM, int WN>
@@ -1733,10 +1741,13 @@ int mm_check(const void* X, int x_dtype, int ldx, const uint8_t* q, const uint16
 int mm_run(const MmPlan& p, const void* X, int x_dtype, int ldx, const uint8_t* q, const uint16_t* scale,
            const uint16_t* min, void* Y, int y_dtype, int ldy, int M, int N, int K, void* ws, hipStream_t s) {
     hipError_t e;
-    if (p.cfg == 2 && (ldx > kTile64MaxStride || K > kTile64MaxStride))  // offsets past 32 bits: the register-staged kernel
-        e = launch_mm<2, 2>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, s);
-    else if (p.cfg == 1)
-        e = launch_mm_lds<4, 4>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, s);
+    if (p.cfg == 1)
+        e = launch_mm_lds<4, 4>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, nullptr, 1, s);
+    else if (p.cfg == 2 && (ldx > kTile64MaxStride || K > kTile64MaxStride))
+        // row offsets past 32 bits: the LDS-staged form of the same tiles and splits (its LDS for kTile64MaxGroups
+        // groups is 160 KiB too); 64-bit offsets would cost the wave-split kernel registers it has not got (246 of 256)
+        e = launch_mm_lds<2, 2>(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, static_cast<float*>(ws),
+                                p.splits, s);
     else if (p.cfg == 2)
         e = launch_mm_tile64(X, x_dtype, ldx, q, scale, min, Y, y_dtype, ldy, M, N, K, static_cast<float*>(ws),
                              p.splits, s);

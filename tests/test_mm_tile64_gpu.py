@@ -53,3 +53,41 @@ def test_tile64_block_shapes(M, N, K, xdt, ydt, dev):
         outs.append(Yw)
     assert torch.equal(outs[0], outs[1])  # the same plan and order of sums
     assert torch.all(ws[nws:] == 0xFF)
+
+
+@pytest.mark.parametrize("M,N,K,ldx", [
+    (2, 70, 82048, 2 ** 25 + 8),           # rows 64 MiB apart, more groups than one block's tables hold
+    (3, 40, 2048 + 128, 2 ** 25 + 8),      # the same stride, few groups, split
+    (1, 3, 2 ** 25 + 128, 2 ** 25 + 128),  # K itself past the 32-bit row offsets
+])
+def test_tile64_wide_strides(M, N, K, ldx, dev):
+    """X rows or code rows further apart than the 32-bit offsets of the wave-split kernel reach"""
+    assert H.mm_plan(M, N, K)[0] == H.MM_TILE64
+    g = torch.Generator(device=dev).manual_seed(K)
+    X = torch.zeros((M - 1) * ldx + K, device=dev, dtype=F16).as_strided((M, K), (ldx, 1))
+    X.copy_(torch.randn(M, K, generator=g, device=dev))
+    q = torch.randint(0, 256, (N, K // 2), generator=g, device=dev, dtype=torch.uint8)
+    s = (torch.rand(N, K // 128, generator=g, device=dev) * 1.9e-2 + 1e-3).half()
+    m = ((torch.randn(N, K // 128, generator=g, device=dev) - 7.5) * s.float()).half()
+    ref, mag = torch.zeros(M, N, device=dev, dtype=torch.float64), torch.zeros(M, N, device=dev, dtype=torch.float64)
+    step = 1 << 20
+    for k in range(0, K, step):
+        c = q[:, k // 2:(k + step) // 2]
+        w = torch.stack((c & 15, c >> 4), -1).reshape(N, -1, 128).double()
+        gs = slice(k // 128, (k + step) // 128)
+        w = (w * s[:, gs].double()[..., None] + m[:, gs].double()[..., None]).reshape(N, -1)
+        x = X[:, k:k + step].double()
+        ref += (x[:, None] * w).sum(-1)
+        mag += (x[:, None] * w).abs().sum(-1)
+    floor = (256 * 2.0 ** -24 * mag).clamp_min(2.0 ** -14)
+    L = H.lib()
+    nws = L.rk_mm_int4_workspace_bytes(M, N, K)
+    ws = torch.empty(max(nws, 16), device=dev, dtype=torch.uint8)
+    for entry in ("ws", "noalloc"):
+        Y = torch.full((M, N), 7.0, device=dev, dtype=F32)
+        args = [H.ptr(X), H.dt(X), ldx, H.ptr(q), H.ptr(s), H.ptr(m), H.ptr(Y), H.dt(Y), N, M, N, K]
+        st = L.rk_mm_int4_g128_ws(*args, H.ptr(ws), nws, H.stream(dev)) if entry == "ws" else \
+            L.rk_mm_int4_g128_noalloc(*args, H.stream(dev))
+        H.check(st, entry)
+        err = ((Y.double() - ref).abs() / torch.maximum(ref.abs(), floor)).max().item()
+        assert err <= 1e-2, (entry, err)
