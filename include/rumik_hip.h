@@ -152,7 +152,7 @@ int rk_mm_int4_g128(const void* X, int x_dtype, int ldx, const uint8_t* q, const
 
 /* The kernel plan rk_mm_int4_g128 (use_workspace = 0) or rk_mm_int4_g128_ws (use_workspace = 1) runs for this
  * shape: *kernel = RK_MM_TILE128 (LDS-staged 128 x 128 tiles), RK_MM_TILE64 (64 x 64 tiles, narrower for few of
- * them, K shared by a block's waves; LDS-staged where ldx or K exceeds 2^25),
+ * them, K shared by a block's waves; LDS-staged for many tiles of a short K, and where ldx or K exceeds 2^25),
  * RK_MM_REGS (register-staged 64 x 64 tiles, for K too long to stage a block's scales in LDS), or, with a
  * workspace only, RK_MM_PREP128 / RK_MM_PREP64 / RK_MM_PREP48 (X prepared once into the workspace in matrix-core
  * fragment order, then blocks of 128 / 64 / 48 rows x 128 columns fed by direct memory-to-LDS copies; chosen when

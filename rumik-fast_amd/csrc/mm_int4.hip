@@ -247,7 +247,10 @@ __global__ __launch_bounds__(512) void mm_int4_lds_kernel(const void* __restrict
                                                           const uint8_t* __restrict__ q, const uint16_t* __restrict__ sc,
                                                           const uint16_t* __restrict__ mn, void* __restrict__ Y,
                                                           int ydt, int ldy, int M, int N, int K,
-                                                          float* __restrict__ part, int splits) {
+                                                          float* __restrict__ part, int nsplit) {
+    // only the 64 x 64 tiles are split: no split arithmetic in the 128 x 128 ones (512 x 22016 x 2048 103.9 us with it,
+    // 100.6 without)
+    const int splits = WM == 2 ? nsplit : 1;
     constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
     constexpr int XCH = BM * 16 / 256;  // 16-byte X chunks per staging thread per step (row r, 8-column block c)
     constexpr int WCH = BN * 4 / 256;   // 16-byte code chunks per staging thread per step (row n, quarter s)
@@ -1549,6 +1552,29 @@ hipError_t launch_mm_stream(const void* X, int xdt, int ldx, const uint8_t* q, c
     return launch_mm_stream_mt<3>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, st);
 }
 
+template <int WM, int WN>
+size_t mm_lds_bytes(int ng) {  // ng: groups of one block
+    constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
+    return 2 * sizeof(MmStage<BM, BN>) + (size_t)BN * ng * 4;
+}
+
+template <int WM, int WN>
+hipError_t launch_mm_lds(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
+                         void* Y, int ydt, int ldy, int M, int N, int K, float* part, int splits, hipStream_t st) {
+    constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
+    const size_t lds = mm_lds_bytes<WM, WN>((K / 128 + splits - 1) / splits);
+    dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits);
+    if (xdt == RK_BF16)
+        hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, true>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt, ldy,
+                           M, N, K, part, splits);
+    else
+        hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, false>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt,
+                           ldy, M, N, K, part, splits);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || splits == 1) return e;
+    return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
+}
+
 // Y (or, split, the partial sums and their ordered sum) of the 64 x 64 tiles: row blocks of at most four m tiles of
 // equal height
 template <int MT, int NT, int W>
@@ -1584,12 +1610,19 @@ hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, c
     const int t16 = (M + 15) / 16, rb = (t16 + 3) / 4, mt = (t16 + rb - 1) / rb, ngb = (K / 128 + splits - 1) / splits;
     const long tiles = (long)((N + 63) / 64) * rb;
     // the narrowest columns that still give every CU at most one block; otherwise 64 columns, by eight waves while one
-    // round takes all blocks and every wave has a group, else by four and two blocks per CU. Measured with 16 / 32 / 64 columns: 69 x 2048
-    // x 2048 6.6 / 7.7 / 10.5 us, 200 x 2048 x 2048 14.2 / 9.7 / 12.8, 512 x 2048 x 2048 26 / 17.3 / 13.1; eight / four
-    // waves: 512 x 2048 x 2048 13.1 / 15.4, 512 x 3072 x 2048 23.9 / 20.0.
+    // round takes all blocks, else by four and two blocks per CU. Measured with 16 / 32 / 64 columns: 69 x 2048 x 2048
+    // 6.6 / 7.7 / 10.5 us, 200 x 2048 x 2048 14.2 / 9.7 / 12.8, 512 x 2048 x 2048 26 / 17.3 / 13.1; eight / four waves:
+    // 512 x 2048 x 2048 13.1 / 15.4, 512 x 3072 x 2048 23.9 / 20.0.
     const long b64 = tiles * splits;
     const int nt = 4 * b64 <= 256 ? 1 : 2 * b64 <= 256 ? 2 : 4;
-    const bool w8 = nt < 4 || (b64 <= 256 && ngb >= 8);
+    // 64 columns and a few groups: too few to pass for a block's start and its sum over waves; the LDS-staged form
+    // shares each group's work among the waves instead. Staged / wave-split, one round of blocks: 256 x 4096 x 128
+    // 5.8 / 7.1 us, x 512 7.8 / 7.8, 64 x 12000 x 768 10.1 / 9.5; more blocks: 200 x 8704 x 512 14.0 / 17.0, 128 x 8200
+    // x 1280 15.1 / 16.4, 1024 x 3500 x 1280 29.0 / 29.4, 128 x 8200 x 1536 17.8 / 16.8. It pads rows to 64: row blocks
+    // of 48 keep the wave-split form past four groups (90 x 17000 x 512 15.0 / 14.9, x 1024 21.5 / 18.8).
+    if (nt == 4 && splits == 1 && K / 128 <= (b64 <= 256 || mt < 4 ? 4 : 10))
+        return launch_mm_lds<2, 2>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, nullptr, 1, st);
+    const bool w8 = nt < 4 || b64 <= 256;
     const int w = w8 && tile64_lds_bytes(mt, nt, 8, ngb) <= kTile64MaxLds ? 8 : 4;
     hipError_t e;
     switch (mt) {
@@ -1598,29 +1631,6 @@ hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, c
         case 3: e = launch_mm_tile64_mt<3>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
         default: e = launch_mm_tile64_mt<4>(nt, w, X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, part, splits, st); break;
     }
-    if (e != hipSuccess || splits == 1) return e;
-    return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
-}
-
-template <int WM, int WN>
-size_t mm_lds_bytes(int ng) {  // ng: groups of one block
-    constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
-    return 2 * sizeof(MmStage<BM, BN>) + (size_t)BN * ng * 4;
-}
-
-template <int WM, int WN>
-hipError_t launch_mm_lds(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
-                         void* Y, int ydt, int ldy, int M, int N, int K, float* part, int splits, hipStream_t st) {
-    constexpr int BM = 2 * WM * 16, BN = 2 * WN * 16;
-    const size_t lds = mm_lds_bytes<WM, WN>((K / 128 + splits - 1) / splits);
-    dim3 grid(((N + BN - 1) / BN) * ((M + BM - 1) / BM) * splits);
-    if (xdt == RK_BF16)
-        hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, true>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt, ldy,
-                           M, N, K, part, splits);
-    else
-        hipLaunchKernelGGL((mm_int4_lds_kernel<WM, WN, false>), grid, dim3(512), lds, st, X, ldx, q, s, m, Y, ydt,
-                           ldy, M, N, K, part, splits);
-    const hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return e;
     return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
 }

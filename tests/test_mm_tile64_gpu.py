@@ -1,5 +1,6 @@
 """The 64 x 64 tile kernel (csrc/mm_int4.hip, RK_MM_TILE64) over its block shapes: 1 .. 4 m tiles, 16 / 32 / 64 columns,
-eight or four waves, whole and split K, waves without a group, ragged rows and columns; against the CPU oracle.
+eight or four waves, whole and split K, waves without a group, the LDS-staged form, ragged rows and columns; against
+the CPU oracle.
 Bar: max relative error <= 1e-2 with the per-output floor max(2^-14, 256 u32 sum_k |X_mk w_nk|), cosine >= 0.9999."""
 import pytest
 import torch
@@ -18,8 +19,12 @@ F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
     (81, 2050, 1920, F16, F16),       # 15 groups: one wave with one group less
     (200, 2040, 2048, BF16, F32),     # 32 columns
     (130, 3100, 1152, F16, F16),      # 64 columns by eight waves, 9 groups
-    (150, 3100, 896, BF16, F16),      # 64 columns by four waves: fewer groups than eight
-    (300, 6000, 384, F16, BF16),      # more blocks than CUs
+    (150, 3100, 896, BF16, F16),      # 64 columns, fewer groups than eight waves
+    (150, 3100, 640, F16, F32),       # the fewest groups the waves share in one round
+    (150, 3100, 512, BF16, F32),      # LDS-staged: one round, four groups
+    (300, 6000, 384, F16, BF16),      # LDS-staged: more blocks than CUs
+    (300, 5701, 1280, BF16, F32),     # LDS-staged: ten groups
+    (300, 5701, 1408, F16, F16),      # 64 columns by four waves, the fewest groups (11)
     (1, 40, 2176, F16, F32),          # 1 m tile, one row, split
     (20, 130, 6400, BF16, F16),       # 2 m tiles, split into narrow columns, N % 4 != 0
     (40, 2052, 11008, F16, F32),      # 3 m tiles, eight splits of 64 columns
