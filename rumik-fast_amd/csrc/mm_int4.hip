@@ -1610,9 +1610,10 @@ hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, c
     const int t16 = (M + 15) / 16, rb = (t16 + 3) / 4, mt = (t16 + rb - 1) / rb, ngb = (K / 128 + splits - 1) / splits;
     const long tiles = (long)((N + 63) / 64) * rb;
     // the narrowest columns that still give every CU at most one block; otherwise 64 columns, by eight waves while one
-    // round takes all blocks, else by four and two blocks per CU. Measured with 16 / 32 / 64 columns: 69 x 2048 x 2048
+    // round takes all blocks, else by four and two blocks per CU while their LDS allows two (four m tiles: up to 64
+    // groups), past that by eight again where they fit (up to 128). Measured with 16 / 32 / 64 columns: 69 x 2048 x 2048
     // 6.6 / 7.7 / 10.5 us, 200 x 2048 x 2048 14.2 / 9.7 / 12.8, 512 x 2048 x 2048 26 / 17.3 / 13.1; eight / four waves:
-    // 512 x 2048 x 2048 13.1 / 15.4, 512 x 3072 x 2048 23.9 / 20.0.
+    // 512 x 2048 x 2048 13.1 / 15.4, 512 x 3072 x 2048 23.9 / 20.0, x 8192 61.2 / 53.4, x 8320 59.6 / 75.0.
     const long b64 = tiles * splits;
     const int nt = 4 * b64 <= 256 ? 1 : 2 * b64 <= 256 ? 2 : 4;
     // 64 columns and a few groups: too few to pass for a block's start and its sum over waves; the LDS-staged form
@@ -1622,7 +1623,7 @@ hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, c
     // of 48 keep the wave-split form past four groups (90 x 17000 x 512 15.0 / 14.9, x 1024 21.5 / 18.8).
     if (nt == 4 && splits == 1 && K / 128 <= (b64 <= 256 || mt < 4 ? 4 : 10))
         return launch_mm_lds<2, 2>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, nullptr, 1, st);
-    const bool w8 = nt < 4 || b64 <= 256;
+    const bool w8 = nt < 4 || b64 <= 256 || 2 * tile64_lds_bytes(mt, 4, 4, ngb) > kTile64MaxLds;
     const int w = w8 && tile64_lds_bytes(mt, nt, 8, ngb) <= kTile64MaxLds ? 8 : 4;
     hipError_t e;
     switch (mt) {

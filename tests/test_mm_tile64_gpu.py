@@ -25,6 +25,7 @@ F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
     (300, 6000, 384, F16, BF16),      # LDS-staged: more blocks than CUs
     (300, 5701, 1280, BF16, F32),     # LDS-staged: ten groups
     (300, 5701, 1408, F16, F16),      # 64 columns by four waves, the fewest groups (11)
+    (300, 3400, 8320, BF16, F32),     # more blocks than CUs, 65 groups: tables too long for two four-wave blocks a CU
     (1, 40, 2176, F16, F32),          # 1 m tile, one row, split
     (20, 130, 6400, BF16, F16),       # 2 m tiles, split into narrow columns, N % 4 != 0
     (40, 2052, 11008, F16, F32),      # 3 m tiles, eight splits of 64 columns
