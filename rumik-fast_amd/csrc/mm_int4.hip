@@ -1687,7 +1687,8 @@ MmPlan mm_plan(int M, int N, int K, int mode);
 // and the reduce launch cost more than they give for short K or few rows (512 x 3072 x 2048 34 us against 24, 128 x
 // 2048 x 11008 32 against 26). Below 64 tiles the splits fill one block of two K ways per CU (200 x 2048 x 11008 29 us,
 // 41 on the 64 x 64 tiles; 300 x 2048 x 11008 36 against 48 with twice the splits); from 64 on two blocks per CU (512 x
-// 2048 x 11008 45 us against 43 for half the splits in two K ways). The workspace holds the prepared X, the partial sums
+// 2048 x 11008 45 us against 43 for half the splits in two K ways), and no more: rounded up, the last few blocks run in
+// a round of their own (104 tiles, 512 x 3328 x 4096: 34.8 us with 4 splits, 45.9 with 5). The workspace holds the prepared X, the partial sums
 // when split, and at least what the tile plan that unaligned scale / min arrays fall back to needs.
 constexpr long kWideMinTiles = 136;
 MmPlan mm_wide_plan(int M, int N, int K) {
@@ -1700,7 +1701,7 @@ MmPlan mm_wide_plan(int M, int N, int K) {
     if (few && (M <= 128 || NG <= 16)) return {-1, 0, 0};
     int S = smin;
     if (few) {
-        const long fill = tiles < 64 ? 256 / tiles : (512 + tiles / 2) / tiles;
+        const long fill = (tiles < 64 ? 256 : 512) / tiles;
         S = std::max<long>(smin, std::min<long>(fill, P / 2));
     }
     if (S > P / 2 || tiles * S < kWideMinTiles) return {-1, 0, 0};

@@ -74,6 +74,16 @@ def test_mm_int4_split_k_plan(M, N, K, splits):
         assert nbytes == (splits * M * N * 4 if splits > 1 else 0)
 
 
+@pytest.mark.parametrize("M,N,K,kernel,splits", [
+    # the wide-wave kernel's splits stay within one round of two blocks per CU
+    (335, 4486, 6912, HL.MM_WIDE128, 4), (512, 3328, 4096, HL.MM_WIDE128, 4), (512, 2432, 11008, HL.MM_WIDE128, 6),
+    (512, 2048, 8192, HL.MM_WIDE128, 8),
+])
+def test_mm_int4_wide_plan_lines(M, N, K, kernel, splits):
+    """Both sides of the lines between the wide-wave kernel, whole or split over K, and the 64 x 64 tiles."""
+    assert HL.mm_plan(M, N, K) == (kernel, splits)
+
+
 def test_mm_int4_ws_rejects_small_workspace():
     lib = HL.lib()
     buf = ctypes.c_void_p(256)  # never dereferenced: validation comes first
