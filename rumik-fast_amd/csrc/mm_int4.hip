@@ -1465,8 +1465,12 @@ struct WideShape {
     int mt, kw;
     long blocks;
 };
+inline int wide_m_tiles(int M) {
+    const int t32 = (M + 31) / 32, rb = (t32 + 3) / 4;
+    return std::max(3, (t32 + rb - 1) / rb);
+}
 inline WideShape wide_shape(int M, int N, int splits) {
-    const int t32 = (M + 31) / 32, rb = (t32 + 3) / 4, mt = std::max(3, (t32 + rb - 1) / rb);
+    const int mt = wide_m_tiles(M);
     const long blocks = (long)((N + kWideCols - 1) / kWideCols) * ((M + 32 * mt - 1) / (32 * mt)) * splits;
     return {mt, blocks <= 256 ? 2 : 1, blocks};
 }
@@ -1575,8 +1579,13 @@ hipError_t launch_mm_lds(const void* X, int xdt, int ldx, const uint8_t* q, cons
     return launch_splitk_reduce(part, splits, Y, ydt, ldy, M, N, st);
 }
 
-// Y (or, split, the partial sums and their ordered sum) of the 64 x 64 tiles: row blocks of at most four m tiles of
-// equal height
+// row blocks of the 64 x 64 tiles: at most four 16-row m tiles, of equal height
+inline int tile64_m_tiles(int M) {
+    const int t16 = (M + 15) / 16, rb = (t16 + 3) / 4;
+    return (t16 + rb - 1) / rb;
+}
+
+// Y (or, split, the partial sums and their ordered sum) of the 64 x 64 tiles
 template <int MT, int NT, int W>
 hipError_t launch_mm_tile64_cfg(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s,
                                 const uint16_t* m, void* Y, int ydt, int ldy, int M, int N, int K, float* part,
@@ -1607,8 +1616,8 @@ hipError_t launch_mm_tile64_mt(int nt, int w, const void* X, int xdt, int ldx, c
 
 hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, const uint16_t* s, const uint16_t* m,
                             void* Y, int ydt, int ldy, int M, int N, int K, float* part, int splits, hipStream_t st) {
-    const int t16 = (M + 15) / 16, rb = (t16 + 3) / 4, mt = (t16 + rb - 1) / rb, ngb = (K / 128 + splits - 1) / splits;
-    const long tiles = (long)((N + 63) / 64) * rb;
+    const int mt = tile64_m_tiles(M), ngb = (K / 128 + splits - 1) / splits;
+    const long tiles = (long)((N + 63) / 64) * ((M + 63) / 64);
     // the narrowest columns that still give every CU at most one block; otherwise 64 columns, by eight waves while one
     // round takes all blocks, else by four and two blocks per CU while their LDS allows two (four m tiles: up to 64
     // groups), past that by eight again where they fit (up to 128). Measured with 16 / 32 / 64 columns: 69 x 2048 x 2048
@@ -1688,21 +1697,27 @@ MmPlan mm_plan(int M, int N, int K, int mode);
 // 2048 x 11008 32 against 26). Below 64 tiles the splits fill one block of two K ways per CU (200 x 2048 x 11008 29 us,
 // 41 on the 64 x 64 tiles; 300 x 2048 x 11008 36 against 48 with twice the splits); from 64 on two blocks per CU (512 x
 // 2048 x 11008 45 us against 43 for half the splits in two K ways), and no more: rounded up, the last few blocks run in
-// a round of their own (104 tiles, 512 x 3328 x 4096: 34.8 us with 4 splits, 45.9 with 5). The workspace holds the prepared X, the partial sums
-// when split, and at least what the tile plan that unaligned scale / min arrays fall back to needs.
-constexpr long kWideMinTiles = 136;
+// a round of their own (104 tiles, 512 x 3328 x 4096: 34.8 us with 4 splits, 45.9 with 5). K too long for one block's
+// tables is split below kWideSplitTiles tiles (64 x 64 tiles / wide: 512 x 4608 x 11008 136 / 96 us, 256 x 9216 x 4096
+// 45.6 / 40.7; from it on other plans take such K, 512 x 5120 x 11008 112 / 98), unless the 64 x 64 tiles are one round
+// of two blocks per CU and pad fewer rows (300 x 6144 x 5120 38 / 44, 130 x 9000 x 4096 28 / 33). The workspace holds the
+// prepared X, the partial sums when split, and at least what the tile plan that unaligned scale / min arrays fall back
+// to needs.
+constexpr long kWideMinTiles = 136, kWideSplitTiles = 160;
 MmPlan mm_wide_plan(int M, int N, int K) {
     const int NG = K / 128, P = NG / 2;
     const long Mp = (M + 15) / 16 * 16;
     const long tiles = (long)((N + 127) / 128) * ((Mp + 127) / 128);
     const int smin = (P + kWideMaxGroups / 2 - 1) / (kWideMaxGroups / 2);
-    const bool few = tiles < kWideMinTiles;
-    if (!few && smin > 1) return {-1, 0, 0};  // enough tiles: no split just to fit the tables
-    if (few && (M <= 128 || NG <= 16)) return {-1, 0, 0};
-    int S = smin;
-    if (few) {
-        const long fill = (tiles < 64 ? 256 : 512) / tiles;
-        S = std::max<long>(smin, std::min<long>(fill, P / 2));
+    const bool whole = tiles >= kWideMinTiles && smin == 1;
+    int S = 1;
+    if (!whole) {
+        if (tiles >= kWideSplitTiles || M <= 128 || NG <= 16) return {-1, 0, 0};
+        const long small = (long)((N + 63) / 64) * ((M + 63) / 64);
+        const int wm = 32 * wide_m_tiles(M), tm = 16 * tile64_m_tiles(M);  // rows of a block
+        const bool padded = (M + wm - 1) / wm * wm > (M + tm - 1) / tm * tm;
+        if (tiles >= kWideMinTiles && small <= 512 && padded) return {-1, 0, 0};
+        S = std::max<long>(smin, std::min<long>((tiles < 64 ? 256 : 512) / tiles, P / 2));
     }
     if (S > P / 2 || tiles * S < kWideMinTiles) return {-1, 0, 0};
     size_t ws = S > 1 ? mm_wide_part_offset(M, K) + (size_t)S * M * N * sizeof(float) : mm_prep_ws_bytes(M, K);
