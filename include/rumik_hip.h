@@ -159,7 +159,7 @@ int rk_mm_int4_g128(const void* X, int x_dtype, int ldx, const uint8_t* q, const
  * the shape has enough column blocks to fill the chip, K is short enough for a block's scale and min rows to sit
  * in LDS, and N * K / 128 is a multiple of 8; RK_MM_WIDE128 is the same for M > 64 with K / 128 even and >= 4:
  * blocks of 128 columns and 96 or 128 rows, a wave per 32 columns, two blocks per CU or one block whose waves share
- * the groups two ways; split over K (*splits > 1) for M > 128 with K / 128 > 16 when the tiles are few), or, for
+ * the groups two ways; split over K (*splits > 1) for M > 128 where the tiles are few and K is long), or, for
  * M <= 48 and K <= 2048 (with or without a workspace),
  * RK_MM_STREAM (X held in registers as matrix-core fragments for the whole launch while 16-column tiles of codes
  * stream past, one block per CU, no workspace);

@@ -1689,20 +1689,28 @@ MmPlan mm_stream_plan(int M, int N, int K, int mode) {
 
 MmPlan mm_plan(int M, int N, int K, int mode);
 
-// The wide-wave plan (cfg 7) for M > 64 and an even group count >= 4. From kWideMinTiles tiles of 128 x 128 on, one
-// block per tile (measured against the 64 x 64 tiles: 149 tiles, 100 x 19000 x 2048, 24 us against 36; 144 tiles, 700 x
-// 3072 x 2048, 26 against 33; 128 tiles, 512 x 4096 x 2048, 25 against 23). Fewer tiles are split over K (whole pairs
-// of groups, >= 4 and <= kWideMaxGroups groups each) for M > 128 and K / 128 > 16: the fp32 partial sums (S x M x N)
-// and the reduce launch cost more than they give for short K or few rows (512 x 3072 x 2048 34 us against 24, 128 x
-// 2048 x 11008 32 against 26). Below 64 tiles the splits fill one block of two K ways per CU (200 x 2048 x 11008 29 us,
-// 41 on the 64 x 64 tiles; 300 x 2048 x 11008 36 against 48 with twice the splits); from 64 on two blocks per CU (512 x
-// 2048 x 11008 45 us against 43 for half the splits in two K ways), and no more: rounded up, the last few blocks run in
-// a round of their own (104 tiles, 512 x 3328 x 4096: 34.8 us with 4 splits, 45.9 with 5). K too long for one block's
-// tables is split below kWideSplitTiles tiles (64 x 64 tiles / wide: 512 x 4608 x 11008 136 / 96 us, 256 x 9216 x 4096
-// 45.6 / 40.7; from it on other plans take such K, 512 x 5120 x 11008 112 / 98), unless the 64 x 64 tiles are one round
-// of two blocks per CU and pad fewer rows (300 x 6144 x 5120 38 / 44, 130 x 9000 x 4096 28 / 33). The workspace holds the
-// prepared X, the partial sums when split, and at least what the tile plan that unaligned scale / min arrays fall back
-// to needs.
+// The wide-wave plan (cfg 7) for M > 64 and an even group count >= 4. All figures: 64 x 64 tiles / wide, in us.
+// From kWideMinTiles tiles of 128 x 128 on one block per tile: 149 tiles, 100 x 19000 x 2048, 32.3 / 24.6; 144 tiles,
+// 700 x 3072 x 2048, 29.1 / 27.0; 135 tiles, 128 x 17280 x 2048, 32.4 / 24.7, but 128 tiles, 512 x 4096 x 2048, 21.7 /
+// 26.0.
+// Fewer tiles are split over K (whole pairs of groups, >= 4 and <= kWideMaxGroups groups each) for M > 128, into one
+// block of two K ways per CU below 64 tiles, from there on into two blocks per CU and no more: rounded up, the last
+// few run in a round of their own (104 tiles, 512 x 3328 x 4096: 34.8 us with 4 splits, 45.9 with 5). The X pre-pass,
+// the fp32 partial sums (S x M x N) and the reduce launch ask for a long K:
+//   * more than 256 of the 64 x 64 tiles (two blocks per CU): past 24 groups (200 x 5000 x 3072 27.0 / 28.5, x 4096
+//     32.3 / 29.5, x 11008 77 / 49; 512 x 3072 x 3072 27 / 31, x 5120 38 / 37), past 20 where the wide blocks have 96
+//     rows and pad none (150 x 6000 x 2304 23.1 / 23.9, x 3072 26.8 / 24.7);
+//   * one round of them, M < 256: past 64 groups (200 x 2048 x 4096 14.2 / 22.8, x 8192 23.5 / 28.1, x 11008 27.5 /
+//     29.1; 129 x 3072 x 8448 27 / 26, x 11008 33 / 29; 150 x 2048 x 11008 26.8 / 25.2), never for 64 or fewer of
+//     them, which split finely (200 x 1024 x 11008 19.7 / 24.8);
+//   * one round, M >= 256: past 16 groups, a line older than the present 64 x 64 tiles, which have since become faster
+//     up to 64 groups (300 x 2048 x 4096 19.7 / 26.1, x 8192 30.5 / 32.1, x 11008 39.2 / 36.8), if the blocks reach
+//     kWideSplitTiles.
+// K too long for one block's tables is split below kWideSplitTiles tiles (512 x 4608 x 11008 114 / 96, 256 x 9216 x
+// 4096 45.6 / 40.7; from it on other plans take such K, 512 x 5120 x 11008 112 / 98), unless the 64 x 64 tiles are one
+// round of two blocks per CU and pad fewer rows (300 x 6144 x 5120 38 / 44, 130 x 9000 x 4096 28 / 33).
+// The workspace holds the prepared X, the partial sums when split, and at least what the tile plan that unaligned
+// scale / min arrays fall back to needs.
 constexpr long kWideMinTiles = 136, kWideSplitTiles = 160;
 MmPlan mm_wide_plan(int M, int N, int K) {
     const int NG = K / 128, P = NG / 2;
@@ -1717,9 +1725,13 @@ MmPlan mm_wide_plan(int M, int N, int K) {
         const int wm = 32 * wide_m_tiles(M), tm = 16 * tile64_m_tiles(M);  // rows of a block
         const bool padded = (M + wm - 1) / wm * wm > (M + tm - 1) / tm * tm;
         if (tiles >= kWideMinTiles && small <= 512 && padded) return {-1, 0, 0};
+        if (tiles < kWideMinTiles) {
+            if (small > 256 ? NG <= (wm == 96 && !padded ? 20 : 24) : M < 256 && (NG <= 64 || small <= 64))
+                return {-1, 0, 0};
+        }
         S = std::max<long>(smin, std::min<long>((tiles < 64 ? 256 : 512) / tiles, P / 2));
     }
-    if (S > P / 2 || tiles * S < kWideMinTiles) return {-1, 0, 0};
+    if (S > P / 2 || (tiles < kWideMinTiles && tiles * S < kWideSplitTiles)) return {-1, 0, 0};
     size_t ws = S > 1 ? mm_wide_part_offset(M, K) + (size_t)S * M * N * sizeof(float) : mm_prep_ws_bytes(M, K);
     ws = std::max(ws, mm_plan(M, N, K, kMmScratch).ws);
     return {7, S, ws};

@@ -78,6 +78,17 @@ def test_mm_int4_split_k_plan(M, N, K, splits):
     # the wide-wave kernel's splits stay within one round of two blocks per CU
     (335, 4486, 6912, HL.MM_WIDE128, 4), (512, 3328, 4096, HL.MM_WIDE128, 4), (512, 2432, 11008, HL.MM_WIDE128, 6),
     (512, 2048, 8192, HL.MM_WIDE128, 8),
+    # M: split from 129 on, up to 255 past 64 groups (one round of 64 x 64 tiles) and not for 64 of them or fewer
+    (128, 2048, 11008, HL.MM_TILE64, 4), (129, 2048, 11008, HL.MM_WIDE128, 8), (129, 2048, 8192, HL.MM_TILE64, 2),
+    (129, 2048, 8448, HL.MM_WIDE128, 8), (200, 2048, 4096, HL.MM_TILE64, 1), (200, 1024, 11008, HL.MM_TILE64, 4),
+    (200, 1088, 11008, HL.MM_WIDE128, 14), (255, 2048, 4096, HL.MM_TILE64, 1), (256, 2048, 4096, HL.MM_WIDE128, 8),
+    # more than one round of 64 x 64 tiles: past 24 groups, past 20 with unpadded 96-row blocks
+    (200, 5000, 3072, HL.MM_TILE64, 1), (200, 5000, 3328, HL.MM_WIDE128, 6), (150, 6000, 2560, HL.MM_TILE64, 1),
+    (150, 6000, 2816, HL.MM_WIDE128, 5), (512, 3328, 3072, HL.MM_TILE64, 1), (512, 3328, 3328, HL.MM_WIDE128, 4),
+    # too few blocks after the split
+    (256, 1024, 4608, HL.MM_TILE64, 1), (256, 1024, 5120, HL.MM_WIDE128, 10),
+    # whole tiles from 136 on
+    (128, 17280, 2048, HL.MM_TILE64, 1), (128, 17281, 2048, HL.MM_WIDE128, 1),
     # K too long for one block's tables: split below 160 tiles, also where whole tiles would do for a shorter K
     (512, 4224, 11008, HL.MM_WIDE128, 4), (512, 4352, 11008, HL.MM_WIDE128, 4), (512, 4608, 11008, HL.MM_WIDE128, 4),
     (512, 4992, 11008, HL.MM_WIDE128, 4), (512, 5120, 11008, HL.MM_TILE64, 1), (512, 4352, 5120, HL.MM_WIDE128, 3),

@@ -18,7 +18,8 @@ F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
     (97, 17420, 1280, F16, F16),     # 4 row tiles with 15 of the last 31 rows absent, two K ways of 5 steps
     (129, 9000, 1024, BF16, F32),    # two row blocks of 3 tiles
     (170, 17000, 512, F16, BF16),    # more blocks than CUs: one K way, 3 row tiles, the fewest groups (4)
-    (200, 2048, 4608, BF16, F16),    # split over K, two K ways of 2 and 3 steps
+    (250, 1030, 8448, BF16, F16),    # split over K, two K ways of 2 and 3 steps
+    (260, 2048, 4608, BF16, F16),    # split, row blocks of 3 tiles, two K ways of 3 and 4 steps
     (250, 1030, 11008, F16, F32),    # split, N % 4 != 0 (the scalar sum over splits)
     (300, 5000, 3328, F16, F16),     # split, one K way
 ])
