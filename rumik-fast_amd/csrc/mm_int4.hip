@@ -1692,7 +1692,10 @@ MmPlan mm_plan(int M, int N, int K, int mode);
 // The wide-wave plan (cfg 7) for M > 64 and an even group count >= 4. All figures: 64 x 64 tiles / wide, in us.
 // From kWideMinTiles tiles of 128 x 128 on one block per tile: 149 tiles, 100 x 19000 x 2048, 32.3 / 24.6; 144 tiles,
 // 700 x 3072 x 2048, 29.1 / 27.0; 135 tiles, 128 x 17280 x 2048, 32.4 / 24.7, but 128 tiles, 512 x 4096 x 2048, 21.7 /
-// 26.0.
+// 26.0. Below kWideSplitTiles not where the 64 x 64 tiles are one round of two blocks per CU and pad fewer rows than
+// 128-row blocks (300 x 6144 x 1024 14.4 / 16.4, 385 x 4400 x 2048 22.5 / 25.3; 96-row ones: up to six groups, 129 x
+// 8800 x 512 10.2 / 10.6), nor for many rows of so few groups that end off 16-byte boundaries, whose pieces share
+// lines (1024 x 2300 x 512 14.2 / 15.9, 1500 x 1500 x 768 18.0 / 19.1; on boundaries 1280 x 1800 x 768 18.6 / 16.1).
 // Fewer tiles are split over K (whole pairs of groups, >= 4 and <= kWideMaxGroups groups each) for M > 128, into one
 // block of two K ways per CU below 64 tiles, from there on into two blocks per CU and no more: rounded up, the last
 // few run in a round of their own (104 tiles, 512 x 3328 x 4096: 34.8 us with 4 splits, 45.9 with 5). The X pre-pass,
@@ -1719,17 +1722,21 @@ MmPlan mm_wide_plan(int M, int N, int K) {
     const int smin = (P + kWideMaxGroups / 2 - 1) / (kWideMaxGroups / 2);
     const bool whole = tiles >= kWideMinTiles && smin == 1;
     int S = 1;
-    if (!whole) {
-        if (tiles >= kWideSplitTiles || M <= 128 || NG <= 16) return {-1, 0, 0};
+    if (!whole || tiles < kWideSplitTiles) {
         const long small = (long)((N + 63) / 64) * ((M + 63) / 64);
         const int wm = 32 * wide_m_tiles(M), tm = 16 * tile64_m_tiles(M);  // rows of a block
         const bool padded = (M + wm - 1) / wm * wm > (M + tm - 1) / tm * tm;
-        if (tiles >= kWideMinTiles && small <= 512 && padded) return {-1, 0, 0};
-        if (tiles < kWideMinTiles) {
-            if (small > 256 ? NG <= (wm == 96 && !padded ? 20 : 24) : M < 256 && (NG <= 64 || small <= 64))
-                return {-1, 0, 0};
+        if (whole) {
+            if (small <= 512 && padded && (wm == 128 || NG <= 6)) return {-1, 0, 0};
+            if (NG <= 6 && M >= 768 && N % 8) return {-1, 0, 0};
+        } else if (tiles >= kWideSplitTiles || M <= 128 || NG <= 16) {
+            return {-1, 0, 0};
+        } else if (tiles >= kWideMinTiles) {
+            if (small <= 512 && padded) return {-1, 0, 0};
+        } else if (small > 256 ? NG <= (wm == 96 && !padded ? 20 : 24) : M < 256 && (NG <= 64 || small <= 64)) {
+            return {-1, 0, 0};
         }
-        S = std::max<long>(smin, std::min<long>((tiles < 64 ? 256 : 512) / tiles, P / 2));
+        if (!whole) S = std::max<long>(smin, std::min<long>((tiles < 64 ? 256 : 512) / tiles, P / 2));
     }
     if (S > P / 2 || (tiles < kWideMinTiles && tiles * S < kWideSplitTiles)) return {-1, 0, 0};
     size_t ws = S > 1 ? mm_wide_part_offset(M, K) + (size_t)S * M * N * sizeof(float) : mm_prep_ws_bytes(M, K);

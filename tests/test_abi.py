@@ -89,6 +89,11 @@ def test_mm_int4_split_k_plan(M, N, K, splits):
     (256, 1024, 4608, HL.MM_TILE64, 1), (256, 1024, 5120, HL.MM_WIDE128, 10),
     # whole tiles from 136 on
     (128, 17280, 2048, HL.MM_TILE64, 1), (128, 17281, 2048, HL.MM_WIDE128, 1),
+    # .. but up to 159 not where one round of 64 x 64 tiles pads fewer rows, or short rows of Y end off 16 bytes
+    (300, 6144, 1024, HL.MM_TILE64, 1), (385, 4400, 3328, HL.MM_TILE64, 1), (129, 8800, 768, HL.MM_TILE64, 1),
+    (129, 8800, 1024, HL.MM_WIDE128, 1), (257, 6200, 1024, HL.MM_WIDE128, 1), (1024, 2300, 768, HL.MM_TILE64, 1),
+    (1024, 2296, 768, HL.MM_WIDE128, 1), (1024, 2300, 1024, HL.MM_WIDE128, 1), (767, 2900, 768, HL.MM_WIDE128, 1),
+    (300, 7000, 1024, HL.MM_WIDE128, 1),
     # K too long for one block's tables: split below 160 tiles, also where whole tiles would do for a shorter K
     (512, 4224, 11008, HL.MM_WIDE128, 4), (512, 4352, 11008, HL.MM_WIDE128, 4), (512, 4608, 11008, HL.MM_WIDE128, 4),
     (512, 4992, 11008, HL.MM_WIDE128, 4), (512, 5120, 11008, HL.MM_TILE64, 1), (512, 4352, 5120, HL.MM_WIDE128, 3),
