@@ -1669,7 +1669,7 @@ constexpr size_t kLdsMax = 160 * 1024;
 // groups); cfg 0 is the register-staged kernel, for K too long to hold one block's scales in LDS.
 struct MmPlan {
     int cfg, splits;
-    size_t ws;  // workspace bytes: fp32 partials (cfg 2 with splits > 1) or the prepared X (cfg 3 - 5)
+    size_t ws;  // workspace bytes: fp32 partials (cfg 2 with splits > 1), the prepared X (cfg 3 - 5), or both (cfg 7)
 };
 
 enum MmMode { kMmPlain = 0, kMmWorkspace = 1, kMmScratch = 2 };  // rk_mm_int4_g128, _ws, _noalloc
@@ -1764,9 +1764,13 @@ MmPlan mm_plan(int M, int N, int K, int mode) {
     if (M > 64 && big >= 256 && mm_lds_bytes<4, 4>(NG) <= kLdsMax) return {1, 1, 0};
     const long small = (long)((N + 63) / 64) * ((M + 63) / 64);
     int splits = 1;
-    // K <= 2048 takes a few steps of eight waves: no split. Up to 7680 only as many splits as fill the chip with
-    // 16-column blocks (their partial sums are the fewest: 48 x 2048 x 5120 10.8 us against 12.8 for eight splits of 64
-    // columns); longer K as many as fill it with 64-column blocks. A split keeps >= 4 groups.
+    // K <= 2048 takes a few steps of eight waves: no split. Up to 60 groups the fewest splits that make 64 blocks of 64
+    // columns, which run as 16-column ones (32-column ones past 64: 33 .. 63 tiles in two splits); longer K takes as
+    // many as fill the chip with 64-column blocks. A split keeps >= 4 groups. Measured, few / many splits, us: 16 tiles
+    // (34 x 1024), K = 5120 8.8 / 10.4, 7680 10.0 / 11.1, 8192 10.1 / 11.4, 11008 11.8 / 12.9; 32 tiles (34 x 2048),
+    // 5120 10.9 / 12.1, 7680 12.8 / 12.2, 11008 14.6 / 13.6; 64 tiles (128 x 2048, unsplit / 4), 5120 14.2 / 15.4, 7680
+    // 17.9 / 17.5, 11008 24.5 / 20.4. Two splits / unsplit: 33 tiles, 64 x 2112 x 2176 10.3 / 8.3, 5120 13.9 / 14.2,
+    // 7680 16.8 / 17.7; 48 tiles, 96 x 1536 x 2176 9.3 / 7.3, 7680 15.2 / 14.7; 63 tiles, 64 x 4032 x 5120 14.8 / 15.3.
     if (allow_ws && small < 256 && NG > 16)
         splits = (int)std::max(1L, std::min(NG <= 60 ? (63 + small) / small : 256 / small, (long)(NG / 4)));
     while (allow_ws && (NG + splits - 1) / splits > kTile64MaxGroups && splits < NG) ++splits;

@@ -54,12 +54,15 @@ def test_version_and_status_strings():
 @pytest.mark.parametrize("M,N,K,splits", [(34, 2048, 11008, 8), (34, 3072, 2048, 1), (128, 2048, 11008, 4),
                                           (200, 33, 11008, 21), (34, 22016, 2048, 1), (512, 2048, 11008, 8),
                                           (512, 22016, 2048, 1), (4, 32, 256, 1), (64, 2048, 11008, 8),
-                                          (5, 200, 4096, 8)])
+                                          (5, 200, 4096, 8), (60, 2048, 2048, 1), (60, 2048, 2176, 2),
+                                          (60, 2048, 7680, 2), (60, 2048, 7808, 8), (64, 4032, 4096, 2),
+                                          (64, 4096, 4096, 1), (64, 1408, 4096, 3), (64, 8192, 11008, 2),
+                                          (64, 8256, 11008, 1)])
 def test_mm_int4_split_k_plan(M, N, K, splits):
-    """fp32 partials only where 64 x 64 output tiles leave CUs idle: splits = min(ceil(256 / tiles), groups / 4);
-    shapes on the prepared-X kernels hold the prepared X instead (the wide-wave kernel split over K, for M >= 256
-    with long K and few 128 x 128 tiles, also its partials: splits = min(round(512 / tiles), groups / 4)), and the
-    stream kernel (M <= 48, K <= 2048) none"""
+    """fp32 partials only where the 64 x 64 output tiles leave CUs idle and K is long: min(256 / tiles, groups / 4) splits
+    past 60 groups, min(ceil(64 / tiles), groups / 4) from 17 on; shapes on the prepared-X kernels hold the prepared X
+    instead (the wide-wave kernel split over K, for M > 128 with long K and few 128 x 128 tiles, also its partials:
+    256 / tiles splits below 64 tiles, 512 / tiles from there on), and the stream kernel (M <= 48, K <= 2048) none"""
     nbytes = HL.lib().rk_mm_int4_workspace_bytes(M, N, K)
     kernel, sp = HL.mm_plan(M, N, K)
     assert sp == splits
@@ -222,10 +225,11 @@ def test_sampler_entry_points_validate_before_any_device_work():
                                           (50, 2048, 11008, HL.MM_TILE64)])
 def test_mm_int4_workspace_plan(M, N, K, kernel):
     """With a workspace, M <= 48 at K <= 2048 takes the stream kernel unless a block's scale / min tables would
-    exceed 2048 entries (very wide N); otherwise shapes with >= 160 column blocks of 128 take the prepared-X kernel
-    (48 / 64 / 128-row blocks by M; for M > 64 the wide-wave kernel when K / 128 is even and >= 4, split over K
-    for M >= 256 with long K and few tiles); too few blocks, K too long for the block's scale tables, or N * K / 128
-    not a multiple of 8 keep the tile plan."""
+    exceed 2048 entries (very wide N); otherwise, for M > 64 and K / 128 even and >= 4, the wide-wave kernel from 136
+    tiles of 128 x 128 on, or split over K for M > 128 with long K and fewer tiles (the lines between are in
+    test_mm_int4_wide_plan_lines); else shapes with >= 160 column blocks of 128 take the prepared-X kernel (48 / 64 /
+    128-row blocks by M); too few blocks, K too long for the block's scale tables, or N * K / 128 not a multiple of 8
+    keep the tile plan."""
     assert HL.mm_plan(M, N, K, use_workspace=True)[0] == kernel
 
 
