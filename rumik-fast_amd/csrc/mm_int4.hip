@@ -1003,13 +1003,27 @@ __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))
         for (int e = 0; e < 16; ++e) acc[mt][e] = 0.f;
     const uint16_t* scol = tsc + (32 * cw + jn) * ngs + kw;
     const uint16_t* mcol = tmn + (32 * cw + jn) * ngs + kw;
+    // the lane's scale, min and row sums of step p + hf (zero past the last), read one pair ahead: the LDS reads and the
+    // centring run under the products
+    uint16_t sr, mr;
+    float xr[MT];
+    auto fetch = [&](int p) {
+        const int st = p + hf, c = min(st, ns - 1);
+        sr = scol[c * KW];
+        mr = mcol[c * KW];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const float x = xsl[(c * KW + kw) * BM + 32 * mt + jn];
+            xr[mt] = st < ns ? x : 0.f;
+        }
+    };
+    fetch(0);
     for (int p = 0; p < ns; p += 2) {
-        const int st = p + hf;
-        const float mv =
-            st < ns ? centred_min(f16_bits_to_f32(mcol[st * KW]), f16_bits_to_f32(scol[st * KW])) : 0.f;
+        const float mv = centred_min(f16_bits_to_f32(mr), f16_bits_to_f32(sr));
         float xa[MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) xa[mt] = st < ns ? xsl[(st * KW + kw) * BM + 32 * mt + jn] : 0.f;
+        for (int mt = 0; mt < MT; ++mt) xa[mt] = xr[mt];
+        fetch(p + 2);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = __builtin_amdgcn_mfma_f32_32x32x2f32(xa[mt], mv, acc[mt], 0, 0, 0);
     }
