@@ -17,6 +17,7 @@ F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
     (96, 17500, 768, BF16, BF16),    # two K ways of 3 steps
     (97, 17420, 1280, F16, F16),     # 4 row tiles with 15 of the last 31 rows absent, two K ways of 5 steps
     (129, 9000, 1024, BF16, F32),    # two row blocks of 3 tiles
+    (131, 17401, 768, BF16, BF16),   # odd N: rows of Y off the 16-byte pieces, one K way
     (170, 17000, 512, F16, BF16),    # more blocks than CUs: one K way, 3 row tiles, the fewest groups (4)
     (250, 1030, 8448, BF16, F16),    # split over K, two K ways of 2 and 3 steps
     (260, 2048, 4608, BF16, F16),    # split, row blocks of 3 tiles, two K ways of 3 and 4 steps
