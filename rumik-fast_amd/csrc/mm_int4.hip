@@ -1651,11 +1651,12 @@ hipError_t launch_mm_tile64(const void* X, int xdt, int ldx, const uint8_t* q, c
     const long b64 = tiles * splits;
     const int nt = 4 * b64 <= 256 ? 1 : 2 * b64 <= 256 ? 2 : 4;
     // 64 columns and a few groups: too few to pass for a block's start and its sum over waves; the LDS-staged form
-    // shares each group's work among the waves instead. Staged / wave-split, one round of blocks: 256 x 4096 x 128
-    // 5.8 / 7.1 us, x 512 7.8 / 7.8, 64 x 12000 x 768 10.1 / 9.5; more blocks: 200 x 8704 x 512 14.0 / 17.0, 128 x 8200
-    // x 1280 15.1 / 16.4, 1024 x 3500 x 1280 29.0 / 29.4, 128 x 8200 x 1536 17.8 / 16.8. It pads rows to 64: row blocks
-    // of 48 keep the wave-split form past four groups (90 x 17000 x 512 15.0 / 14.9, x 1024 21.5 / 18.8).
-    if (nt == 4 && splits == 1 && K / 128 <= (b64 <= 256 || mt < 4 ? 4 : 10))
+    // shares each group's work among the waves instead. Staged / wave-split, one round of blocks: 256 x 4096 x 128 5.8
+    // / 7.1 us, x 640 8.65 / 8.8, 987 x 525 x 640 8.4 / 9.2, 64 x 12000 x 768 10.1 / 9.5; more blocks: 200 x 8704 x
+    // 512 14.0 / 17.0, 128 x 8200 x 1280 15.1 / 16.4, 1024 x 3500 x 1280 29.0 / 29.4, 128 x 8200 x 1536 17.8 / 16.8.
+    // It pads rows to 64: row blocks of 48 keep the wave-split form past five groups (90 x 17000 x 640 16.7 / 17.2, x
+    // 1024 21.5 / 18.8).
+    if (nt == 4 && splits == 1 && K / 128 <= (b64 <= 256 || mt < 4 ? 5 : 10))
         return launch_mm_lds<2, 2>(X, xdt, ldx, q, s, m, Y, ydt, ldy, M, N, K, nullptr, 1, st);
     const bool w8 = nt < 4 || b64 <= 256 || 2 * tile64_lds_bytes(mt, 4, 4, ngb) > kTile64MaxLds;
     const int w = w8 && tile64_lds_bytes(mt, nt, 8, ngb) <= kTile64MaxLds ? 8 : 4;

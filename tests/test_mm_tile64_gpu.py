@@ -20,8 +20,8 @@ F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
     (200, 2040, 2048, BF16, F32),     # 32 columns
     (130, 3100, 1152, F16, F16),      # 64 columns by eight waves, 9 groups
     (150, 3100, 896, BF16, F16),      # 64 columns, fewer groups than eight waves
-    (150, 3100, 640, F16, F32),       # the fewest groups the waves share in one round
-    (150, 3100, 512, BF16, F32),      # LDS-staged: one round, four groups
+    (150, 3100, 768, F16, F32),       # the fewest groups the waves share in one round
+    (150, 3100, 640, BF16, F32),      # LDS-staged: one round, five groups
     (300, 6000, 384, F16, BF16),      # LDS-staged: more blocks than CUs
     (300, 5701, 1280, BF16, F32),     # LDS-staged: ten groups
     (300, 5701, 1408, F16, F16),      # 64 columns by four waves, the fewest groups (11)
