@@ -1737,7 +1737,9 @@ MmPlan mm_plan(int M, int N, int K, int mode);
 //     kWideSplitTiles.
 // K too long for one block's tables is split below kWideSplitTiles tiles (512 x 4608 x 11008 114 / 96, 256 x 9216 x
 // 4096 45.6 / 40.7; from it on other plans take such K, 512 x 5120 x 11008 112 / 98), unless the 64 x 64 tiles are one
-// round of two blocks per CU and pad fewer rows (300 x 6144 x 5120 38 / 44, 130 x 9000 x 4096 28 / 33).
+// round of two blocks per CU and either pad fewer rows (300 x 6144 x 5120 38 / 44, 130 x 9000 x 4096 28 / 33) or have
+// at most 48 groups (181 x 9886 x 3840 33.4 / 38.7, x 4608 37.6 / 41.6, x 6400 48.9 / 50.2; 150 x 9500 x 4608 36.6 /
+// 37.5, x 6400 47.8 / 45.3).
 // The workspace holds the prepared X, the partial sums when split, and at least what the tile plan that unaligned
 // scale / min arrays fall back to needs.
 constexpr long kWideMinTiles = 136, kWideSplitTiles = 160;
@@ -1758,7 +1760,7 @@ MmPlan mm_wide_plan(int M, int N, int K) {
         } else if (tiles >= kWideSplitTiles || M <= 128 || NG <= 16) {
             return {-1, 0, 0};
         } else if (tiles >= kWideMinTiles) {
-            if (small <= 512 && padded) return {-1, 0, 0};
+            if (small <= 512 && (padded || NG <= 48)) return {-1, 0, 0};
         } else if (small > 256 ? NG <= (wm == 96 && !padded ? 20 : 24) : M < 256 && (NG <= 64 || small <= 64)) {
             return {-1, 0, 0};
         }

@@ -102,6 +102,7 @@ def test_mm_int4_split_k_plan(M, N, K, splits):
     (512, 4992, 11008, HL.MM_WIDE128, 4), (512, 5120, 11008, HL.MM_TILE64, 1), (512, 4352, 5120, HL.MM_WIDE128, 3),
     (384, 6144, 4096, HL.MM_WIDE128, 3), (512, 4352, 3328, HL.MM_WIDE128, 1), (512, 4352, 3584, HL.MM_WIDE128, 3),
     (256, 9000, 16384, HL.MM_WIDE128, 5), (300, 6144, 5120, HL.MM_TILE64, 1), (128, 17500, 5120, HL.MM_TILE64, 1),
+    (181, 9886, 6144, HL.MM_TILE64, 1), (181, 9886, 6400, HL.MM_WIDE128, 3), (181, 9886, 3328, HL.MM_WIDE128, 1),
 ])
 def test_mm_int4_wide_plan_lines(M, N, K, kernel, splits):
     """Both sides of the lines between the wide-wave kernel, whole or split over K, and the 64 x 64 tiles."""
