@@ -163,8 +163,8 @@ int rk_mm_int4_g128(const void* X, int x_dtype, int ldx, const uint8_t* q, const
  * M <= 48 and K <= 2048 (with or without a workspace),
  * RK_MM_STREAM (X held in registers as matrix-core fragments for the whole launch while 16-column tiles of codes
  * stream past, one block per CU, no workspace);
- * *splits = the number of K splits (1 = none; > 1 only with a workspace). Host-only query, no GPU needed; RK_ERR_SHAPE for sizes rk_mm_int4_g128 rejects. Part of the
- * mm_int4 drop-in (reference kernels/mm_int4.py:59-73 picks its Triton tile from BM / BN); the reference has no
+ * *splits = the number of K splits (1 = none; > 1 only with a workspace). Host-only query, no GPU needed;
+ * RK_ERR_SHAPE for sizes rk_mm_int4_g128 rejects. Part of the mm_int4 drop-in (reference kernels/mm_int4.py:59-73 picks its Triton tile from BM / BN); the reference has no
  * plan query. */
 #define RK_MM_REGS 0
 #define RK_MM_TILE128 1

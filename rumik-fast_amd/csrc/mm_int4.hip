@@ -906,13 +906,13 @@ RK_DEV void wide_barrier() {
 // aligned scale / min arrays; the host checks all of them.
 constexpr int kWideMaxGroups = 26;  // LDS: 2 x 128 x 26 fp16 of tables beside the 66 KiB area (KW = 1) stay <= 80 KiB
 
+// two waves per SIMD: 256 VGPRs (<4, 2> takes 236, no form spills)
 template <int MT, int KW>
-__global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))) void mm_int4_wide_kernel(const uint4* __restrict__ Xp,
-                                                              const float* __restrict__ xsg, int Mp,
-                                                              const uint8_t* __restrict__ q,
-                                                              const uint16_t* __restrict__ sc,
-                                                              const uint16_t* __restrict__ mn, void* __restrict__ Y,
-                                                              int ydt, int ldy, int M, int N, int K, int splits) {
+__global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void mm_int4_wide_kernel(const uint4* __restrict__ Xp, const float* __restrict__ xsg, int Mp,
+                         const uint8_t* __restrict__ q, const uint16_t* __restrict__ sc,
+                         const uint16_t* __restrict__ mn, void* __restrict__ Y, int ydt, int ldy, int M, int N, int K,
+                         int splits) {
     constexpr int BM = 32 * MT, BN = kWideCols, CW = 4, SLOT = wide_slot_bytes(MT);
     constexpr int XC = MT * 8 / CW;  // X copies of a wave per step (its K way's slot is copied by the way's four waves)
     extern __shared__ __align__(16) uint8_t smem[];
@@ -1110,8 +1110,8 @@ __global__ __launch_bounds__(256 * KW) __attribute__((amdgpu_waves_per_eu(2, 2))
     const bool vec_ok = (((uintptr_t)Y | (size_t)ldy * (ydt == RK_F32 ? 4 : 2)) & (ydt == RK_F32 ? 15 : 7)) == 0;
     const int r0 = kw * (BM / KW), n0 = nb + 32 * cw;
     if (!vec_ok) {
-        // rows off those boundaries: single elements, 32 consecutive ones of two rows at a time (in pieces of 8 per lane
-        // every store touched 16 rows: 512 x 25089 x 2048 99.7 us, 88.2 so; 963 x 11005 x 1024 61.9 / 48.9)
+        // rows off those boundaries: single elements, 32 consecutive ones of two rows at a time (in pieces of 8 per
+        // lane every store touched 16 rows: 512 x 25089 x 2048 99.7 us, 88.2 so; 963 x 11005 x 1024 61.9 / 48.9)
 #pragma unroll 4
         for (int i = 0; i < BM / KW / 2; ++i) {
             const int r = r0 + 2 * i + hf, m = mb + r, n = n0 + jn;

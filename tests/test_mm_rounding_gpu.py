@@ -1,5 +1,5 @@
-"""Rounding of the int4 prefill product (csrc/mm_int4.hip), fp32 outputs against 64 bits: a kernel that adds the groups' min
-terms apart from their scaled products must be no further off than the group-by-group order of the reference
+"""Rounding of the int4 prefill product (csrc/mm_int4.hip), fp32 outputs against 64 bits: a kernel that adds the groups'
+min terms apart from their scaled products must be no further off than the group-by-group order of the reference
 (kernels/mm_int4.py:24-46: acc += scale * dot + min * rowsum, all fp32), also for activations with a mean, where the
 two sums cancel."""
 import numpy as np
